@@ -400,7 +400,8 @@ def work(case):
 
 def tolerance(case):
     """About four times what the path differs by from itself in 64 bits (sums of products; bf16 operands rounded as
-    the path rounds them).  Seen, largest of all outputs: 1.1e-6 and 1e-5 (the layers), 4e-8 and 2e-7 (densities), 2.1e-5 and 4e-3 (bf16: a projection on a rounding boundary)."""
+    the path rounds them).  Seen, largest of all outputs: 1.1e-6 and 1e-5 (the layers), 4e-8 and 2e-7 (densities),
+    2.1e-5 and 4e-3 (bf16: a projection on a rounding boundary)."""
     if case["kind"] == "search":
         return "exact"
     if case["kind"] == "density":
