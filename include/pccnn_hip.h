@@ -486,7 +486,7 @@ int pccnn_mcconv_weight_var(const float *pts, const float *pdf, const float *fea
                             void *workspace, size_t workspace_bytes, void *stream);
 
 /* ---- dense contraction --------------------------------------------------
- * The fp32 MFMA GEMM the convolutions use for the [M, K*Cin] x [K*Cin, Cout]
+ * The fp32 GEMM (matrix cores) the convolutions use for the [M, K*Cin] x [K*Cin, Cout]
  * contraction (torch::matmul at pccnn_lib_ops/pcconvs/kpconv.cu:56-57,90-96 and
  * mcconv.cu:64-68,111-120), exposed for tests and benchmarks.
  * C[batch][rows,cols] = op(A) * op(B) with inner size `inner`; row-major storage,

@@ -228,6 +228,12 @@ size_t pccnn_scan_tmp_elems(int64_t n);
 int pccnn_scan_inclusive_i32(const int32_t *in, int32_t *out, int64_t n, int clamp_max, int32_t *tmp,
                              hipStream_t stream, int64_t *total64_out = nullptr);
 
+// The split of a product's reduction that pccnn_gemm_f32 is fastest with, for a split-k workspace of that many floats,
+// and the sum of split-k partial products that both contractions end with (gemm.hip).
+int pccnn_gemm_f32_split(int64_t rows, int64_t cols, int64_t inner, int batch, size_t workspace_floats);
+int pccnn_splitk_reduce(const float *partial, float *c, int64_t rows, int64_t cols, int64_t ldc, int64_t stride_c,
+                        int split_k, int batch, hipStream_t s);
+
 // bf16 contraction (gemm_bf16.hip), used by conv.hip.
 extern "C" int pccnn_f32_to_bf16(const float *src, uint16_t *dst, int64_t count, void *stream);
 extern "C" int pccnn_gemm_bf16(const uint16_t *a, const uint16_t *b, float *c, int64_t rows, int64_t cols,

@@ -1,5 +1,5 @@
 // KPConv / MCConv: basis projection and neighbor gather-aggregate (forward and backward), plus
-// the host entry points that chain them with the fp32 MFMA contraction.
+// the host entry points that chain them with the fp32 contraction.
 //
 // Forward, per sample s:  P[s][f][k] = sum over the pairs t of s of  F[n_t][f] * w[t][k]
 //   * one wavefront per (sample, block of 64 input features): lane l owns feature f = 64*fb + l
@@ -1271,7 +1271,12 @@ static int conv_validate(const char *who, int64_t n, int64_t m, int64_t t, int d
     return PCCNN_OK;
 }
 
-#define CONV_SPLIT_K 64
+// floats that the split of d_weights = P^T x dOut over the samples may take for its partial products
+static size_t conv_splitk_floats(int c_in, int k, int c_out)
+{
+    const size_t weights = (size_t)c_in * k * c_out;
+    return weights * 64 > (1u << 20) ? weights * 64 : (1u << 20);
+}
 
 extern "C" size_t pccnn_conv_workspace_bytes(int64_t m, int64_t t, int c_in, int k, int c_out, int backward)
 {
@@ -1283,7 +1288,7 @@ extern "C" size_t pccnn_conv_workspace_bytes(int64_t m, int64_t t, int c_in, int
     // (a forward call that keeps no projection may run fused and then needs room for the repacked weights only)
     if (!backward) return proj + w16 + pair_b + pccnn_conv_fused_workspace_bytes(c_in, k, c_out) + 256;
     size_t basis_g = pccnn_align((size_t)t * k * sizeof(float));
-    size_t splitk = pccnn_align((size_t)CONV_SPLIT_K * c_in * k * c_out * sizeof(float));
+    size_t splitk = pccnn_align(conv_splitk_floats(c_in, k, c_out) * sizeof(float));
     size_t partials = pccnn_align(((size_t)PARAM_ROWS + PARAM_REDUCE_GROUPS) * 256 * sizeof(float));
     size_t scaled = pccnn_align((size_t)m * c_out * sizeof(float));
     size_t pair_g = pccnn_align((size_t)t * 4 * sizeof(float));
@@ -1301,22 +1306,19 @@ extern "C" size_t pccnn_conv_workspace_bytes_deterministic(int64_t n, int64_t m,
            pccnn_align((size_t)t * c_in * sizeof(float)) + by_point_index_bytes(n, t) + 256;
 }
 
-// out[m, c_out] = P[m, c_in*k] x W, with the feature axis split over num_mlps independent
-// weight blocks (num_mlps == 1 is the plain product).
-// Split of the sample dimension for d_weights = P^T x dOut, whose output ([K*Cin, Cout]) has few tiles: enough
-// workgroups for about four per CU, but (fp32 operands) at least 2048 samples each, so that the partial sums
-// written and summed again stay small beside the product itself.
-static int conv_split_k(int64_t inner, int64_t co, int num_mlps, int64_t m, bool bf16)
+// Split of the sample dimension for d_weights = P^T x dOut with bf16 operands, whose output ([K*Cin, Cout]) has few
+// tiles: bound by its operand traffic, so about four workgroups per CU, with at least 128 samples each.
+static int conv_split_k_bf16(int64_t inner, int64_t co, int num_mlps, int64_t m, size_t workspace_floats)
 {
-    if (m < 4096) return 1;
-    if (bf16) return CONV_SPLIT_K;      // bound by its operand traffic: the more workgroups in flight the better
-    const int64_t tiles = pccnn_ceil_div(inner, 64) * pccnn_ceil_div(co, 128) * num_mlps;
-    int64_t split = 1024 / tiles;
-    if (split > m / 2048) split = m / 2048;
-    if (split > CONV_SPLIT_K) split = CONV_SPLIT_K;
-    return (int)(split < 1 ? 1 : split);
+    int64_t split = pccnn_ceil_div(1024, pccnn_ceil_div(inner, 64) * pccnn_ceil_div(co, 128) * num_mlps);
+    const int64_t room = (int64_t)(workspace_floats / ((size_t)inner * co * num_mlps));
+    if (split > m / 128) split = m / 128;
+    if (split > room) split = room;
+    return split < 1 ? 1 : (int)split;
 }
 
+// out[m, c_out] = P[m, c_in*k] x W, with the feature axis split over num_mlps independent
+// weight blocks (num_mlps == 1 is the plain product).
 static int contraction_fwd(const float *proj, const float *weights, float *out, int64_t m, int c_in, int k,
                            int num_mlps, int c_out, hipStream_t s)
 {
@@ -1487,7 +1489,7 @@ static int conv_backward(ConvGeom g, const float *feats, const float *weights, c
     float *proj_ws = arena.take<float>(proj_elems);
     float *d_proj = arena.take<float>(proj_elems);
     float *basis_g = arena.take<float>((size_t)g.t * g.k);
-    size_t splitk_elems = (size_t)CONV_SPLIT_K * g.c_in * g.k * c_out;
+    const size_t splitk_elems = conv_splitk_floats(g.c_in, g.k, c_out);
     float *splitk = arena.take<float>(splitk_elems);
     float *scaled_grads = arena.take<float>((size_t)g.m * c_out);
     float *pair_grads = arena.take<float>((size_t)g.t * 4);
@@ -1535,7 +1537,8 @@ static int conv_backward(ConvGeom g, const float *feats, const float *weights, c
             if ((rc = launch_proj_fwd<BASIS>(g, feats, proj_ws, s, bf16)) != PCCNN_OK) return rc;
             proj = proj_ws;
         }
-        const int split = conv_split_k(inner, co, num_mlps, g.m, bf16);
+        const int split = bf16 ? conv_split_k_bf16(inner, co, num_mlps, g.m, splitk_elems)
+                               : pccnn_gemm_f32_split(inner, co, g.m, num_mlps, splitk_elems);
         if (bf16)
             rc = pccnn_gemm_bf16((const uint16_t *)proj, g16, d_weights, inner, co, g.m, 1, 0, (int64_t)g.c_in * g.k,
                                  c_out, co, num_mlps, inner, co, inner * co, split, splitk,

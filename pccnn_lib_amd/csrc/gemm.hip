@@ -1,26 +1,49 @@
-// fp32 GEMM on the CDNA matrix cores (v_mfma_f32_32x32x2_f32), used for the
-// [M, K*Cin] x [K*Cin, Cout] contraction of the convolutions and its two transposes.
+// fp32 GEMM on the CDNA matrix cores: the [M, K*Cin] x [K*Cin, Cout] contraction of the convolutions and its two
+// transposes.
 //
-// Two kernels.  gemm_f32_full_tiles_kernel takes the products whose tiles are all full (the shapes of the
-// convolutions: thousands of rows, a multiple of 128 columns): its k loop holds nothing but MFMAs, four or three
-// 16-byte global loads, as many 16-byte LDS stores and the fragment reads.  gemm_f32_mfma_kernel takes everything
-// else (edge tiles, odd leading dimensions, very short reductions) with bounds checks where a tile needs them.
+// Two kernels.  gemm_f32_split_kernel takes the products that can fill the chip: every fp32 operand is carried as
+// three bf16 terms and multiplied on the bf16 matrix pipe (v_mfma_f32_32x32x16_bf16), whose rate is sixteen times
+// that of the fp32 matrix instructions and beside which vector instructions run (beside the fp32 ones they do not).
+// gemm_f32_short_kernel takes the small ones, which are bound by latency, on the fp32 matrix instructions.  Split-K
+// writes partial products to a workspace that a further kernel sums in a fixed order.
 //
-// Common to both: workgroup tile 128 x 128 (4 wavefronts as 2 x 2, each a 64 x 64 block of 2 x 2 MFMA tiles) or,
-// when the grid would otherwise be too small to fill the chip, 64 x 128 (1 x 4 wavefronts of 64 x 32); inner step
-// 16; operand tiles double-buffered in LDS, the next tile's global loads issued before the current tile's MFMAs,
-// one barrier per step.  Split-K writes partial products to a workspace that a second kernel sums in a fixed order.
+// The three terms lose nothing: x = h1 + h2 + h3 exactly, with h1 = x rounded to bf16 (8 significant bits), h2 the
+// rest rounded to bf16, h3 what is left (at most 8 bits of the 24 remain).  A product of two terms is exact in fp32
+// (16 bits), and the sums are fp32.  Of the nine products of a pair x y the three smallest, h2 h3', h3 h2' and
+// h3 h3', are left out: together at most 2^-24 |x y|, what rounding the product once to fp32 loses.  Error against
+// float64, relative to the result's norm, this kernel / the fp32 matrix instructions: reduction of 128: 1.6e-7 /
+// 2.0e-7, 1024: 4.9e-7 / 5.7e-7, 1920: 2.6e-7 / 7.8e-7, 3855 of 65 536: 3.9e-7 / 1.1e-6.
+//
+// Measured, before (128 x 128 and 64 x 128 tiles of fp32 matrix instructions) and now, us: 65 536 x 128 x 1024 138 ->
+// 109, its transposes 165 -> 121 and 149 -> 119; 65 536 x 256 x 1920 483 -> 368 (175 TFLOP/s; the fp32 instructions'
+// peak is 157), transposes 522 -> 370 and 515 -> 391; 120 000 x 64 x 1920 541 -> 247; 37 675 x 96 x 720 84 -> 55;
+// 40 000 x 205 x 645 (odd leading dimension) 207 -> 91; 24 x 33 x 7327 138 -> 10; 346 x 256 x 1024 51 -> 11.
+// The large ones are bound by the matrix pipe at the clock that its power allows (counters: 54 % of the cycles at
+// 1.96 GHz; the library's bf16 product reaches 1.34 PFLOP/s on this part, this kernel 1.05 of the six products).
 #include <type_traits>
 
 #include "common.h"
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));      // dword-aligned 16-byte access
+typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-#define GT_M 128
-#define GT_N 128
-#define GT_K 16
-#define GT_LD 130          // LDS row stride (floats): conflict-free transposing stores, 8-byte aligned rows
+#define GS_K 32            // reduction elements per step of the split kernel
+#define GS_PLANES 3
+// Operands are scaled by 2^16 (exact) on their way into terms and results back by 2^-32: a third term of the smallest
+// normal number then still is a bf16 number, and even subnormal operands are carried exactly.  What overflows on the
+// way (operands from 2^112, sums from 2^96) is computed again at the end of the kernel.
+#define GS_SCALE 65536.0f
+// Longer reductions keep the sum of the largest products h1 h1' apart from that of the five smaller ones, so that the
+// large sum is rounded once and not six times per 16 elements (error at 1920: 6.8e-7 -> 2.6e-7 of the result's norm).
+// The second sum costs registers and with them a wavefront per SIMD where the reduction is short (65 536 x 1024 x 128,
+// B transposed: 121 -> 130 us), and there one sum is as precise as it need be.
+#define GS_ONE_SUM 1024
+#define GS_STAGE_LD 36     // floats per row of a staged output tile
 
 struct GemmArgs {
     const float *a, *b;
@@ -29,9 +52,7 @@ struct GemmArgs {
     int64_t lda, ldb, ldc;
     int64_t stride_a, stride_b, stride_c;
     int split_k;
-    int64_t k_chunk;       // inner elements per split (multiple of GT_K)
-    int aligned;           // pointers, leading dimensions and batch strides allow float4 loads
-    int whole_units;       // aligned, and no float4 unit of a tile straddles the edge of its operand
+    int64_t k_chunk;       // inner elements per split
     int tiles_x, tiles_y;  // workgroup tiles along the columns / rows
     int64_t total_wg;      // tiles_x * tiles_y * batch * split_k
 };
@@ -43,456 +64,559 @@ struct GemmArgs {
 // row tile (or, with one column tile, their B chunk), which is then fetched from HBM by one XCD, once.
 #define GEMM_XCDS 8
 
-// Global -> registers for one 128 x 16 operand tile.  `KCONTIG`: the reduction index is the
-// contiguous one in memory (element (x, k) at p[x * ld + k]); otherwise element (x, k) at p[k * ld + x].
-// MODE 1: the tile is fully inside the matrix and 16-byte aligned, so it is read with float4 loads and no checks;
-// MODE 2: float4 loads, a unit outside the matrix reads as zeros (the host checks that no unit straddles an edge:
-// the extents along the units are multiples of 4); MODE 0: element by element.
-template <bool KCONTIG, int MODE, int TILE_X>
-__device__ __forceinline__ void tile_load(const float *__restrict__ p, int64_t ld, int64_t x0, int64_t x_end,
-                                          int64_t k0, int64_t k_end, float4 (&r)[TILE_X / 64 * (GT_K / 16)])
-{
-#pragma unroll
-    for (int i = 0; i < TILE_X / 64 * (GT_K / 16); ++i) {
-        const int idx = threadIdx.x + 256 * i;
-        int64_t x, k;
-        if (KCONTIG) { x = x0 + idx / (GT_K / 4); k = k0 + (idx % (GT_K / 4)) * 4; }
-        else { k = k0 + idx / (TILE_X / 4); x = x0 + (idx % (TILE_X / 4)) * 4; }
-        if (MODE == 1) {
-            r[i] = KCONTIG ? *(const float4 *)(p + x * ld + k) : *(const float4 *)(p + k * ld + x);
-        } else if (MODE == 2) {
-            r[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (x < x_end && k < k_end)
-                r[i] = KCONTIG ? *(const float4 *)(p + x * ld + k) : *(const float4 *)(p + k * ld + x);
-        } else {
-            float v[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int64_t xx = KCONTIG ? x : x + c;
-                const int64_t kk = KCONTIG ? k + c : k;
-                v[c] = (xx < x_end && kk < k_end) ? (KCONTIG ? p[xx * ld + kk] : p[kk * ld + xx]) : 0.0f;
-            }
-            r[i] = make_float4(v[0], v[1], v[2], v[3]);
-        }
-    }
-}
+struct GemmTile {
+    int64_t bm, bn, k_begin, k_end;
+    int batch, split;
+    bool valid;
+};
 
-template <bool KCONTIG, int TILE_X>
-__device__ __forceinline__ void tile_store(float (*lds)[GT_LD], const float4 (&r)[TILE_X / 64 * (GT_K / 16)])
+template <int BM, int BN>
+__device__ __forceinline__ GemmTile gemm_tile(const GemmArgs &g)
 {
-#pragma unroll
-    for (int i = 0; i < TILE_X / 64 * (GT_K / 16); ++i) {
-        const int idx = threadIdx.x + 256 * i;
-        if (KCONTIG) {
-            const int x = idx / (GT_K / 4), k = (idx % (GT_K / 4)) * 4;
-            lds[k + 0][x] = r[i].x;
-            lds[k + 1][x] = r[i].y;
-            lds[k + 2][x] = r[i].z;
-            lds[k + 3][x] = r[i].w;
-        } else {
-            const int k = idx / (TILE_X / 4), x = (idx % (TILE_X / 4)) * 4;
-            *(float2 *)&lds[k][x] = make_float2(r[i].x, r[i].y);
-            *(float2 *)&lds[k][x + 2] = make_float2(r[i].z, r[i].w);
-        }
-    }
-}
-
-// The k loop of one workgroup tile.  Global loads run two or three tiles ahead of the MFMAs (one or two register
-// sets, then the free LDS buffer); inside a tile the LDS fragments of sub-step ks+1 are read before the MFMAs of
-// sub-step ks are issued, so the matrix pipe never waits on an LDS round trip.
-template <bool AT, bool BT, int MODE, int BM>
-__device__ __forceinline__ void gemm_tile_loop(const GemmArgs &g, const float *__restrict__ a,
-                                               const float *__restrict__ b, int64_t bm, int64_t bn, int64_t k_begin,
-                                               int64_t k_end, float (*As)[GT_K][GT_LD], float (*Bs)[GT_K][GT_LD],
-                                               floatx16 (&acc)[2][BM / 64])
-{
-    constexpr int WN = 4 / (BM / 64);                               // wavefronts along the columns
-    constexpr int TN = BM / 64;                                     // 32-column MFMA tiles per wavefront
-    const int lane = pccnn_lane();
-    const int wave = threadIdx.x >> 6;
-    const int wm = wave / WN, wn = wave % WN;
-    const int frag_k = lane >> 5, frag_c = lane & 31;
-    constexpr int NA = BM / 64 * (GT_K / 16), NB = 2 * (GT_K / 16);
-    // 64-row tiles on the fast path travel in two register sets (tile j in set j & 1), so every global load has
-    // two whole steps of MFMAs to arrive (3 - 4 % on the products of 65 536 x 1024 x 128).  The 128-row tiles keep
-    // one set (AHEAD = 2): with two they pass 128 registers, which halves the waves per SIMD and costs 9 %; so does
-    // the bounds-checked path of edge tiles.
-    constexpr bool DEEP = MODE == 1 && BM == 64;
-    constexpr int AHEAD = DEEP ? 3 : 2;
-    float4 ra0[NA], rb0[NB], ra1[DEEP ? NA : 1], rb1[DEEP ? NB : 1];
-    const int64_t nk = (k_end - k_begin + GT_K - 1) / GT_K;
-    // A stored [rows, inner] (AT = false) has the reduction index contiguous; B stored
-    // [inner, cols] (BT = false) has the column index contiguous.
-    if (nk > 0) {
-        tile_load<!AT, MODE, BM>(a, g.lda, bm, g.rows, k_begin, k_end, ra0);
-        tile_load<BT, MODE, GT_N>(b, g.ldb, bn, g.cols, k_begin, k_end, rb0);
-        tile_store<!AT, BM>(As[0], ra0);
-        tile_store<BT, GT_N>(Bs[0], rb0);
-    }
-    if constexpr (DEEP) {
-        if (nk > 1) {
-            tile_load<!AT, MODE, BM>(a, g.lda, bm, g.rows, k_begin + GT_K, k_end, ra1);
-            tile_load<BT, MODE, GT_N>(b, g.ldb, bn, g.cols, k_begin + GT_K, k_end, rb1);
-        }
-        if (nk > 2) {
-            tile_load<!AT, MODE, BM>(a, g.lda, bm, g.rows, k_begin + 2 * GT_K, k_end, ra0);
-            tile_load<BT, MODE, GT_N>(b, g.ldb, bn, g.cols, k_begin + 2 * GT_K, k_end, rb0);
-        }
-    } else if (nk > 1) {
-        tile_load<!AT, MODE, BM>(a, g.lda, bm, g.rows, k_begin + GT_K, k_end, ra0);
-        tile_load<BT, MODE, GT_N>(b, g.ldb, bn, g.cols, k_begin + GT_K, k_end, rb0);
-    }
-    __syncthreads();
-    // One step: the MFMAs of tile kt from LDS buffer kt & 1.  Behind the first of them tile kt+1, which sits in
-    // the register set (ra, rb), is parked in the other LDS buffer (free since the barrier that ended step kt-1)
-    // and the same registers take the loads of tile kt+AHEAD.
-    auto step = [&](int64_t kt, float4 (&ra)[NA], float4 (&rb)[NB]) {
-        const int buf = (int)(kt & 1);
-        float fa[2][2], fb[2][TN];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) fa[0][i] = As[buf][frag_k][wm * 64 + i * 32 + frag_c];
-#pragma unroll
-        for (int j = 0; j < TN; ++j) fb[0][j] = Bs[buf][frag_k][wn * (32 * TN) + j * 32 + frag_c];
-#pragma unroll
-        for (int ks = 0; ks < GT_K / 2; ++ks) {
-            const int cur = ks & 1, nxt = cur ^ 1;
-            if (ks + 1 < GT_K / 2) {
-                const int kr = 2 * (ks + 1) + frag_k;
-#pragma unroll
-                for (int i = 0; i < 2; ++i) fa[nxt][i] = As[buf][kr][wm * 64 + i * 32 + frag_c];
-#pragma unroll
-                for (int j = 0; j < TN; ++j) fb[nxt][j] = Bs[buf][kr][wn * (32 * TN) + j * 32 + frag_c];
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[cur][i], fb[cur][j], acc[i][j], 0, 0, 0);
-            if (ks == 0) {
-                // behind the first MFMAs of the step, so the matrix pipe is busy while this wave moves data
-                if (kt + 1 < nk) {
-                    tile_store<!AT, BM>(As[buf ^ 1], ra);
-                    tile_store<BT, GT_N>(Bs[buf ^ 1], rb);
-                }
-                if (kt + AHEAD < nk) {
-                    const int64_t k0 = k_begin + (kt + AHEAD) * GT_K;
-                    tile_load<!AT, MODE, BM>(a, g.lda, bm, g.rows, k0, k_end, ra);
-                    tile_load<BT, MODE, GT_N>(b, g.ldb, bn, g.cols, k0, k_end, rb);
-                }
-            }
-            // keep the order written above in the instruction stream: the fragment reads of the next sub-step go
-            // out before this sub-step's MFMAs, so their LDS latency is covered by the matrix pipe
-            if (ks + 1 < GT_K / 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 2 * TN, 0);
-        }
-        __syncthreads();
-    };
-    if constexpr (DEEP) {
-        for (int64_t kt = 0; kt < nk; kt += 2) {
-            step(kt, ra1, rb1);                                     // tile kt+1 (odd) travels in set 1
-            if (kt + 1 < nk) step(kt + 1, ra0, rb0);                // tile kt+2 (even) in set 0
-        }
-    } else {
-        for (int64_t kt = 0; kt < nk; ++kt) step(kt, ra0, rb0);
-    }
-}
-
-template <bool AT, bool BT, int BM>
-__global__ void __launch_bounds__(256)
-gemm_f32_mfma_kernel(GemmArgs g, float *__restrict__ partial)
-{
-    __shared__ __attribute__((aligned(16))) float As[2][GT_K][GT_LD];
-    __shared__ __attribute__((aligned(16))) float Bs[2][GT_K][GT_LD];
-    constexpr int WN = 4 / (BM / 64);
-    constexpr int TN = BM / 64;
-
-    const int lane = pccnn_lane();
-    const int wave = threadIdx.x >> 6;
-    const int wm = wave / WN, wn = wave % WN;
+    GemmTile t;
     const int64_t per_xcd = (int64_t)gridDim.x / GEMM_XCDS;
     const int64_t tile = (int64_t)(blockIdx.x % GEMM_XCDS) * per_xcd + blockIdx.x / GEMM_XCDS;
-    if (tile >= g.total_wg) return;                                 // padding of the launch
+    t.valid = tile < g.total_wg;                                    // false: padding of the launch
     const int tx = (int)(tile % g.tiles_x);
     const int ty = (int)((tile / g.tiles_x) % g.tiles_y);
     const int tz = (int)(tile / ((int64_t)g.tiles_x * g.tiles_y));
-    const int batch = tz / g.split_k;
-    const int split = tz % g.split_k;
-    const int64_t bm = (int64_t)ty * BM;
-    const int64_t bn = (int64_t)tx * GT_N;
-    const float *a = g.a + (int64_t)batch * g.stride_a;
-    const float *b = g.b + (int64_t)batch * g.stride_b;
-    const int64_t k_begin = (int64_t)split * g.k_chunk;
-    const int64_t k_end = (k_begin + g.k_chunk < g.inner) ? k_begin + g.k_chunk : g.inner;
-    const bool fast = g.aligned && (bm + BM <= g.rows) && (bn + GT_N <= g.cols) && ((k_end - k_begin) % GT_K == 0);
+    t.batch = tz / g.split_k;
+    t.split = tz % g.split_k;
+    t.bm = (int64_t)ty * BM;
+    t.bn = (int64_t)tx * BN;
+    t.k_begin = (int64_t)t.split * g.k_chunk;
+    t.k_end = (t.k_begin + g.k_chunk < g.inner) ? t.k_begin + g.k_chunk : g.inner;
+    return t;
+}
 
-    floatx16 acc[2][TN];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-    if (fast) gemm_tile_loop<AT, BT, 1, BM>(g, a, b, bm, bn, k_begin, k_end, As, Bs, acc);
-    else if (g.whole_units) gemm_tile_loop<AT, BT, 2, BM>(g, a, b, bm, bn, k_begin, k_end, As, Bs, acc);
-    else gemm_tile_loop<AT, BT, 0, BM>(g, a, b, bm, bn, k_begin, k_end, As, Bs, acc);
-
-    // Accumulator layout of the 32x32 MFMA: register v of lane l holds
-    // row 8*(v/4) + 4*(l/32) + v%4, column l%32 of the tile.
-    float *cbase;
-    int64_t ldc;
+__device__ __forceinline__ float *gemm_output(const GemmArgs &g, const GemmTile &t, float *partial, int64_t &ldc)
+{
     if (g.split_k > 1) {
-        cbase = partial + ((int64_t)batch * g.split_k + split) * g.rows * g.cols;
         ldc = g.cols;
-    } else {
-        cbase = g.c + (int64_t)batch * g.stride_c;
-        ldc = g.ldc;
+        return partial + ((int64_t)t.batch * g.split_k + t.split) * g.rows * g.cols;
     }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int64_t col = bn + wn * (32 * TN) + j * 32 + (lane & 31);
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int64_t row = bm + wm * 64 + i * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
-                if (row < g.rows && col < g.cols) cbase[row * ldc + col] = acc[i][j][v];
-            }
-        }
+    ldc = g.ldc;
+    return g.c + (int64_t)t.batch * g.stride_c;
+}
+
+// One element of the product by fp32 multiply-adds, in order.
+__device__ __forceinline__ float gemm_dot(const float *__restrict__ a, const float *__restrict__ b, int64_t a_step,
+                                          int64_t b_step, int64_t count)
+{
+    float s = 0.0f;
+    for (int64_t k = 0; k < count && s == s; ++k) s = fmaf(a[k * a_step], b[k * b_step], s);
+    return s;
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// The kernel for full tiles (rows % BM == 0, cols % 128 == 0, every k range a multiple of 16, 16-byte alignment).
-// On this part vector-ALU and memory instructions are not hidden behind the MFMAs of the other wavefronts of a
-// SIMD: a k step costs its MFMA cycles plus about 4 cycles per vector instruction and about 60 per global load.
-// The loop therefore carries no address arithmetic at all:
-//  * global loads take a uniform base (advanced with scalar adds) and a 32-bit lane offset computed once;
-//  * the k loop is unrolled over the two LDS buffers, so every LDS address is a register plus an immediate;
-//  * an operand whose reduction index is contiguous in memory ("KC": A [rows, inner], B [cols, inner]) keeps its
-//    16-byte chunks (4 k) whole: one ds_write_b128 per chunk, and the lane that feeds row r of a 32-row MFMA tile
-//    reads a whole chunk back (ds_read_b128).  Chunk c of row r sits in slot c ^ swz(r), so that the lanes of one
-//    LDS pass hit distinct banks.  An operand whose row / column index is contiguous ("XC") lands k-major; the k
-//    rows with (k >> 2) & 1 set are rotated by 32 elements so that the two halves of a wavefront, which read
-//    different k, use different banks;
-//  * which k a lane multiplies in which MFMA is free as long as both operands agree: lane half h takes
-//    k = 4 (2 j + h) + e in the e-th MFMA of group j (e = 0..3, j = 0..1 per 16-k tile).
-// One barrier per k step, in its middle: behind it the buffer of the current tile is free and the next tile is
-// complete, whose first fragments are requested before the second half of the step's MFMAs.
-__device__ __forceinline__ int gl_row_swz(int r) { return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1); }
+// Split kernel.  Workgroup: 4 wavefronts, WM x WN of them, each TM x TN MFMA tiles of 32 x 32; inner step 32.
+//
+// An operand tile of X rows (or columns) sits in LDS as 16-byte units of 8 consecutive k of one row, one plane per
+// term: unit (term, k / 8, x) in slot gs_slot(x, k / 8).  A fragment of the MFMA is one unit per lane, 32 consecutive
+// x: one ds_read_b128 without bank conflicts.  A thread makes whole units: it loads 8 k of a row (XC with 96 or more
+// rows: of two neighboring rows) and splits them in registers.
+//   KC (reduction index contiguous in memory): unit u = (x = u / 4, k / 8 = u % 4), two 16-byte loads;
+//   XC (row / column index contiguous): unit u = (k / 8 = u / (X / W), x = W (u % (X / W))), eight loads of W floats.
+// The wide loads are dword-aligned: any leading dimension.  Rows past the edge read the last row (their results are
+// not stored); an XC pair that straddles the edge reads the next row's first element; the last step of a reduction
+// that is not whole is loaded element by element, with zeros past its end, so nothing outside the operands is touched.
+//
+// One LDS buffer and two barriers per step, the next step's loads in flight in registers: the two or three workgroups
+// of a CU fill each other's gaps.  Tried and not faster: two steps of loads ahead (no difference); two LDS buffers of
+// 16 with one barrier and the split between the MFMAs of the same wavefront (361 against 364 us at 65 536 x 256 x
+// 1920, slower on narrow tiles and spilling with both operands XC); 256 x 128 tiles (324 there, 118 against 107 at
+// 65 536 x 128 x 1024, 483 against 368 with both operands XC).
+__device__ __forceinline__ int gs_slot(int x, int k8) { return x ^ ((x >> 3) & 1) ^ (k8 << 1); }
 
-// byte offset, from the tile's origin, of the 16-byte chunk this lane loads first; its i-th load is the same lane
-// offset from a base moved on by gl_load_delta() elements
-template <bool KC, int X>
-__device__ __forceinline__ unsigned gl_lane_offset(int wave, int lane, int64_t ld)
+__device__ __forceinline__ uint32_t gs_pack(float lo, float hi)
 {
-    const int q = wave * (X / 64);
-    if (KC) {
-        const int row = q * 16 + (lane >> 2);
-        return (unsigned)((row * ld + (((lane & 3) ^ gl_row_swz(row)) << 2)) * 4);
-    }
-    const int e = q * 64 + lane;
-    const int k = e / (X / 4), pos = e % (X / 4);
-    return (unsigned)((k * ld + ((pos ^ (((k >> 2) & 1) << 3)) << 2)) * 4);
+    const floatx2 v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
-template <bool KC, int X>
-__device__ __forceinline__ int64_t gl_load_delta(int64_t ld) { return KC ? 16 * ld : (256 / X) * ld; }
 
-template <bool AT, bool BT, int BM>
-__global__ void __launch_bounds__(256)
-gemm_f32_full_tiles_kernel(GemmArgs g, float *__restrict__ partial)
+// The three terms of eight values, packed in order.
+__device__ __forceinline__ void gs_split(const float (&x)[8], uint4 (&term)[GS_PLANES])
 {
-    constexpr bool AKC = !AT, BKC = BT;
-    constexpr int WN = 4 / (BM / 64);                               // wavefronts along the columns
-    constexpr int TN = BM / 64;                                     // 32-column MFMA tiles per wavefront
-    constexpr int NA = BM / 64, NB = GT_N / 64;                     // 16-byte loads per lane and k tile
-    __shared__ __attribute__((aligned(16))) float As[2][BM * GT_K];
-    __shared__ __attribute__((aligned(16))) float Bs[2][GT_N * GT_K];
+    uint32_t t[GS_PLANES][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float lo = x[2 * i] * GS_SCALE, hi = x[2 * i + 1] * GS_SCALE;
+#pragma unroll
+        for (int p = 0; p < GS_PLANES; ++p) {
+            const uint32_t w = gs_pack(lo, hi);
+            t[p][i] = w;
+            if (p + 1 < GS_PLANES) {
+                lo -= __uint_as_float(w << 16);
+                hi -= __uint_as_float(w & 0xffff0000u);
+            }
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < GS_PLANES; ++p) term[p] = make_uint4(t[p][0], t[p][1], t[p][2], t[p][3]);
+}
 
+template <bool KC, int X> struct SplitOperand {
+    static constexpr int W = (!KC && X >= 96) ? 2 : 1;              // rows per unit load
+    static constexpr int UNITS = X * (GS_K / 8) / W;
+    static constexpr int PASSES = (UNITS + 255) / 256;
+    const float *base;                                              // uniform: origin of the current step
+    int64_t ld;
+    unsigned off[PASSES];                                           // this thread's units, in bytes
+    int x_left;                                                     // rows of the operand from the tile's first on
+    struct Regs { float v[PASSES][8 * W]; };
+
+    __device__ __forceinline__ static bool active(int i) { return UNITS % 256 == 0 || (int)threadIdx.x + 256 * i < UNITS; }
+    __device__ __forceinline__ static void unit(int i, int &x, int &k8)
+    {
+        const int u = threadIdx.x + 256 * i;
+        if (KC) { x = u / (GS_K / 8); k8 = u % (GS_K / 8); }
+        else { k8 = u / (X / W); x = (u % (X / W)) * W; }
+    }
+    __device__ __forceinline__ void init(const float *origin, int64_t ld_, int64_t x0, int64_t x_end, int64_t k0)
+    {
+        ld = ld_;
+        base = origin + (KC ? x0 * ld + k0 : k0 * ld + x0);
+        x_left = (int)((x_end - x0) < X ? (x_end - x0) : X);
+#pragma unroll
+        for (int i = 0; i < PASSES; ++i) {
+            int x, k8;
+            unit(i, x, k8);
+            const unsigned xc = (unsigned)(x < x_left ? x : x_left - 1), kk = (unsigned)(k8 * 8);
+            off[i] = (KC ? xc * (unsigned)ld + kk : kk * (unsigned)ld + xc) * 4u;
+        }
+    }
+    // the step at `base`, which moves on
+    __device__ __forceinline__ void load(Regs &r)
+    {
+#pragma unroll
+        for (int i = 0; i < PASSES; ++i) {
+            if (!active(i)) break;
+            if (KC) {
+                const floatx4u lo = *(const floatx4u *)((const char *)base + off[i]);
+                const floatx4u hi = *(const floatx4u *)((const char *)(base + 4) + off[i]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { r.v[i][e] = lo[e]; r.v[i][4 + e] = hi[e]; }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const char *p = (const char *)(base + e * ld) + off[i];
+                    if (W == 2) {
+                        const floatx2u q = *(const floatx2u *)p;
+                        r.v[i][2 * e] = q[0];
+                        r.v[i][2 * e + W - 1] = q[1];
+                    } else {
+                        r.v[i][e] = *(const float *)p;
+                    }
+                }
+            }
+        }
+        base += KC ? GS_K : GS_K * ld;
+    }
+    // the last step: k_left elements of the reduction, zeros past them
+    __device__ __forceinline__ void load_last(Regs &r, int k_left)
+    {
+#pragma unroll
+        for (int i = 0; i < PASSES; ++i) {
+            if (!active(i)) break;
+            int x, k8;
+            unit(i, x, k8);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int k = k8 * 8 + e;
+                const bool in = k < k_left;
+                const int64_t kc = in ? k : k_left - 1;
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    const int64_t xc = x + w < x_left ? x + w : x_left - 1;
+                    const float q = base[KC ? xc * ld + kc : kc * ld + xc];
+                    r.v[i][e * W + w] = in ? q : 0.0f;
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ static void park(const Regs &r, uint4 (*lds)[GS_K / 8][X])
+    {
+#pragma unroll
+        for (int i = 0; i < PASSES; ++i) {
+            if (!active(i)) break;
+            int x, k8;
+            unit(i, x, k8);
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                float q[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) q[e] = r.v[i][e * W + w];
+                uint4 term[GS_PLANES];
+                gs_split(q, term);
+#pragma unroll
+                for (int p = 0; p < GS_PLANES; ++p) lds[p][k8][gs_slot(x + w, k8)] = term[p];
+            }
+        }
+    }
+};
+
+template <bool AT, bool BT, int WM, int WN, int TM, int TN, bool LOW>
+__global__ void __launch_bounds__(256, 2)
+gemm_f32_split_kernel(GemmArgs g, float *__restrict__ partial)
+{
+    constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
+    __shared__ uint4 lds[GS_PLANES * (GS_K / 8) * (BM + BN)];
+    uint4 (*As)[GS_K / 8][BM] = (uint4 (*)[GS_K / 8][BM])lds;
+    uint4 (*Bs)[GS_K / 8][BN] = (uint4 (*)[GS_K / 8][BN])(lds + GS_PLANES * (GS_K / 8) * BM);
     const int lane = pccnn_lane();
     const int wave = threadIdx.x >> 6;
     const int wm = wave / WN, wn = wave % WN;
     const int r = lane & 31, h = lane >> 5;
-    const int64_t per_xcd = (int64_t)gridDim.x / GEMM_XCDS;
-    const int64_t tile = (int64_t)(blockIdx.x % GEMM_XCDS) * per_xcd + blockIdx.x / GEMM_XCDS;
-    if (tile >= g.total_wg) return;
-    const int tx = (int)(tile % g.tiles_x);
-    const int ty = (int)((tile / g.tiles_x) % g.tiles_y);
-    const int tz = (int)(tile / ((int64_t)g.tiles_x * g.tiles_y));
-    const int batch = tz / g.split_k;
-    const int split = tz % g.split_k;
-    const int64_t bm = (int64_t)ty * BM;
-    const int64_t bn = (int64_t)tx * GT_N;
-    const int64_t k_begin = (int64_t)split * g.k_chunk;
-    const int64_t k_end = (k_begin + g.k_chunk < g.inner) ? k_begin + g.k_chunk : g.inner;
-    const int64_t nk = (k_end - k_begin) / GT_K;
-    // uniform: the origin of the current k tile of either operand
-    const float *a_tile = g.a + (int64_t)batch * g.stride_a + (AKC ? bm * g.lda + k_begin : k_begin * g.lda + bm);
-    const float *b_tile = g.b + (int64_t)batch * g.stride_b + (BKC ? bn * g.ldb + k_begin : k_begin * g.ldb + bn);
-    const int64_t a_step = AKC ? GT_K : GT_K * g.lda;
-    const int64_t b_step = BKC ? GT_K : GT_K * g.ldb;
-    const unsigned a_lane = gl_lane_offset<AKC, BM>(wave, lane, g.lda);
-    const unsigned b_lane = gl_lane_offset<BKC, GT_N>(wave, lane, g.ldb);
-    const int64_t a_delta = gl_load_delta<AKC, BM>(g.lda), b_delta = gl_load_delta<BKC, GT_N>(g.ldb);
+    const GemmTile t = gemm_tile<BM, BN>(g);
+    if (!t.valid) return;
+    const float *a = g.a + (int64_t)t.batch * g.stride_a;
+    const float *b = g.b + (int64_t)t.batch * g.stride_b;
 
-    floatx16 acc[2][TN];
+    floatx16 acc[TM][TN], low[LOW ? TM : 1][LOW ? TN : 1];          // LOW: h1 h1', and the five smaller products
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-    // where this lane parks its loads (floats from the start of a buffer) and where its fragments are
-    const int a_park = (wave * NA * 64 + lane) * 4, b_park = (wave * NB * 64 + lane) * 4;
-    int a_off[2], b_off[TN];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int x = (BM == 64 ? 0 : wm * 64) + i * 32 + r;
-        a_off[i] = AKC ? x * GT_K + ((h ^ gl_row_swz(r)) << 2) : (4 * h) * BM + (x ^ (h << 5));
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int x = wn * (32 * TN) + j * 32 + r;
-        b_off[j] = BKC ? x * GT_K + ((h ^ gl_row_swz(r)) << 2) : (4 * h) * GT_N + (x ^ (h << 5));
-    }
-
-    // A tile is requested one k step before it is parked in LDS.  (Two register sets, two steps ahead, were
-    // measured and are not faster.)
-    floatx4 ra[NA], rb[NB];
-    auto load_tile = [&]() __attribute__((always_inline)) {         // the tile at (a_tile, b_tile), which move on
-#pragma unroll
-        for (int i = 0; i < NA; ++i) ra[i] = *(const floatx4 *)((const char *)(a_tile + i * a_delta) + a_lane);
-#pragma unroll
-        for (int i = 0; i < NB; ++i) rb[i] = *(const floatx4 *)((const char *)(b_tile + i * b_delta) + b_lane);
-        a_tile += a_step;
-        b_tile += b_step;
-    };
-    auto park_tile = [&](float *as, float *bs) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < NA; ++i) *(floatx4 *)(as + a_park + i * 256) = ra[i];
-#pragma unroll
-        for (int i = 0; i < NB; ++i) *(floatx4 *)(bs + b_park + i * 256) = rb[i];
-    };
-    float fa[2][2][4], fb[2][TN][4];                                // [half j of the tile][MFMA tile][e]
-    auto read_frags = [&](const float *as, const float *bs, int j) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            if (AKC) {
-                // chunk 2 j + h sits in slot (2 j + h) ^ swz = (h ^ swz) ^ 2 j
-                const floatx4 v = *(const floatx4 *)(as + (a_off[i] ^ (j << 3)));
-                fa[j][i][0] = v.x; fa[j][i][1] = v.y; fa[j][i][2] = v.z; fa[j][i][3] = v.w;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) fa[j][i][e] = as[a_off[i] + (8 * j + e) * BM];
+            for (int v = 0; v < 16; ++v) {
+                acc[i][j][v] = 0.0f;
+                if (LOW) low[i][j][v] = 0.0f;
             }
-        }
-#pragma unroll
-        for (int t = 0; t < TN; ++t) {
-            if (BKC) {
-                const floatx4 v = *(const floatx4 *)(bs + (b_off[t] ^ (j << 3)));
-                fb[j][t][0] = v.x; fb[j][t][1] = v.y; fb[j][t][2] = v.z; fb[j][t][3] = v.w;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) fb[j][t][e] = bs[b_off[t] + (8 * j + e) * GT_N];
-            }
-        }
-    };
-    auto mfmas = [&](int j) __attribute__((always_inline)) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int t = 0; t < TN; ++t)
-                    acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j][t][e], fa[j][i][e], acc[i][t], 0, 0, 0);
-    };
+
+    SplitOperand<!AT, BM> oa;
+    SplitOperand<BT, BN> ob;
+    oa.init(a, g.lda, t.bm, g.rows, t.k_begin);
+    ob.init(b, g.ldb, t.bn, g.cols, t.k_begin);
+    typename SplitOperand<!AT, BM>::Regs va;
+    typename SplitOperand<BT, BN>::Regs vb;
+    const int64_t nk = (t.k_end - t.k_begin + GS_K - 1) / GS_K;
+    // the last step needs no checks when it is whole and no pair of rows straddles an edge
+    const bool whole = (t.k_end - t.k_begin) % GS_K == 0 && (SplitOperand<!AT, BM>::W == 1 || g.rows % 2 == 0) &&
+                       (SplitOperand<BT, BN>::W == 1 || g.cols % 2 == 0);
+    const int nf = (int)(whole ? nk : nk - 1);                      // steps loaded without checks
     // this wave's LDS traffic is complete, then everyone's (the global loads stay in flight)
     auto lds_barrier = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    // One k tile, whose first half is in the registers on entry: `cur` is its buffer, `nxt` takes tile kt + 1
-    // (in the registers since the previous step) before the barrier.
-    auto step = [&](auto cur_c, int64_t kt, auto full) __attribute__((always_inline)) {
-        constexpr int cur = decltype(cur_c)::value, nxt = cur ^ 1;
-        read_frags(As[cur], Bs[cur], 1);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (full || kt + 1 < nk) {
-            park_tile(As[nxt], Bs[nxt]);
-            lds_barrier();
-            if (full || kt + 2 < nk) load_tile();
-            read_frags(As[nxt], Bs[nxt], 0);
+    auto multiply = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int ks = 0; ks < GS_K / 16; ++ks) {
+            const int k8 = 2 * ks + h;
+            bf16x8 fa[GS_PLANES][TM], fb[GS_PLANES][TN];
+#pragma unroll
+            for (int p = 0; p < GS_PLANES; ++p) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    fa[p][i] = __builtin_bit_cast(bf16x8, As[p][k8][gs_slot(wm * (TM * 32) + i * 32 + r, k8)]);
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    fb[p][j] = __builtin_bit_cast(bf16x8, Bs[p][k8][gs_slot(wn * (TN * 32) + j * 32 + r, k8)]);
+            }
+            // the operands are swapped (see the store below)
+            constexpr int PA[6] = {0, 2, 1, 0, 1, 0}, PB[6] = {2, 0, 1, 1, 0, 0};
+#pragma unroll
+            for (int n = 0; n < 6; ++n)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        floatx16 &sum = LOW && n < 5 ? low[LOW ? i : 0][LOW ? j : 0] : acc[i][j];
+                        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[PB[n]][j], fa[PA[n]][i], sum, 0, 0, 0);
+                    }
         }
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(1);
-        __builtin_amdgcn_sched_barrier(0);
     };
-
-    if (nk > 0) {
-        load_tile();
-        park_tile(As[0], Bs[0]);
-        if (nk > 1) load_tile();
+    if (nf > 0) {
+        oa.load(va);
+        ob.load(vb);
+    }
+    for (int kt = 0; kt < nf; ++kt) {
+        if (kt > 0) lds_barrier();                                  // everyone has read the previous step
+        SplitOperand<!AT, BM>::park(va, As);
+        SplitOperand<BT, BN>::park(vb, Bs);
         lds_barrier();
-        read_frags(As[0], Bs[0], 0);
+        if (kt + 1 < nf) {
+            oa.load(va);
+            ob.load(vb);
+        }
+        multiply();
     }
-    int64_t kt = 0;
-    for (; kt + 3 < nk; kt += 2) {                                  // every tile the two steps ask for exists
-        step(std::integral_constant<int, 0>(), kt, std::true_type());
-        step(std::integral_constant<int, 1>(), kt + 1, std::true_type());
-    }
-    for (; kt < nk; kt += 2) {
-        step(std::integral_constant<int, 0>(), kt, std::false_type());
-        if (kt + 1 < nk) step(std::integral_constant<int, 1>(), kt + 1, std::false_type());
+    if (nf < nk) {                                                  // the last step, element by element
+        const int k_left = (int)(t.k_end - t.k_begin - (int64_t)nf * GS_K);
+        oa.load_last(va, k_left);
+        ob.load_last(vb, k_left);
+        lds_barrier();
+        SplitOperand<!AT, BM>::park(va, As);
+        SplitOperand<BT, BN>::park(vb, Bs);
+        lds_barrier();
+        multiply();
     }
 
-    float *cbase;
+    // With the operands swapped a tile of the accumulator is the transpose of the output tile: lane l holds output
+    // row l % 32 and, in registers 4 g .. 4 g + 3, the four consecutive columns 8 g + 4 (l / 32) + 0..3.  A tile goes
+    // through the wavefront's own piece of LDS so that a store writes eight whole 128-byte rows.
     int64_t ldc;
-    if (g.split_k > 1) {
-        cbase = partial + ((int64_t)batch * g.split_k + split) * g.rows * g.cols;
-        ldc = g.cols;
-    } else {
-        cbase = g.c + (int64_t)batch * g.stride_c;
-        ldc = g.ldc;
-    }
-    // The MFMAs ran with the operands swapped (B fragment as the 32 x 2 operand), so a tile of the accumulator is
-    // the transpose of the output tile: lane l holds output row l % 32 and, in registers 4 g .. 4 g + 3, the four
-    // consecutive columns 8 g + 4 (l / 32) + 0..3: one 16-byte store each, a quarter of the store instructions
-    // that one register per store would need.
+    float *cbase = gemm_output(g, t, partial, ldc);
+    lds_barrier();                                                  // the fragments of the last step have been read
+    float *stage = (float *)lds + wave * (32 * GS_STAGE_LD);
+    const int srow = lane >> 3, scol = (lane & 7) * 4;
+    bool finite = true;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int64_t row = bm + (BM == 64 ? 0 : wm * 64) + i * 32 + r;
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int t = 0; t < TN; ++t)
+        for (int j = 0; j < TN; ++j) {
 #pragma unroll
             for (int gq = 0; gq < 4; ++gq) {
-                const int64_t col = bn + wn * (32 * TN) + t * 32 + 8 * gq + 4 * h;
                 floatx4 v;
-                v[0] = acc[i][t][4 * gq + 0]; v[1] = acc[i][t][4 * gq + 1];
-                v[2] = acc[i][t][4 * gq + 2]; v[3] = acc[i][t][4 * gq + 3];
-                *(floatx4 *)(cbase + row * ldc + col) = v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = acc[i][j][4 * gq + e];
+                    if (LOW) v[e] += low[LOW ? i : 0][LOW ? j : 0][4 * gq + e];
+                    v[e] *= 1.0f / (GS_SCALE * GS_SCALE);
+                    finite = finite && fabsf(v[e]) <= 3.402823466e38f;
+                }
+                *(floatx4 *)(stage + r * GS_STAGE_LD + 8 * gq + 4 * h) = v;
             }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const int64_t col = t.bn + (wn * TN + j) * 32 + scol;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int64_t row = t.bm + (wm * TM + i) * 32 + q * 8 + srow;
+                const floatx4 v = *(const floatx4 *)(stage + (q * 8 + srow) * GS_STAGE_LD + scol);
+                if (row < g.rows && col + 4 <= g.cols) {
+                    *(floatx4u *)(cbase + row * ldc + col) = v;
+                } else if (row < g.rows) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (col + e < g.cols) cbase[row * ldc + col + e] = v[e];
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    // An infinite operand (or one that rounds up to infinity as bf16) makes its terms' products infinity times zero.
+    // Results that are not finite are computed again by plain multiply-adds, which give what fp32 arithmetic gives.
+    if (__any(!finite)) {
+        __threadfence_block();
+        for (int e = 0; e < TM * TN * 16; ++e) {
+            const int tile = e / 16, v = e % 16;
+            const int64_t row = t.bm + (wm * TM + tile / TN) * 32 + r;
+            const int64_t col = t.bn + (wn * TN + tile % TN) * 32 + 8 * (v / 4) + 4 * h + v % 4;
+            if (row >= g.rows || col >= g.cols || fabsf(cbase[row * ldc + col]) <= 3.402823466e38f) continue;
+            cbase[row * ldc + col] = gemm_dot(a + (AT ? t.k_begin * g.lda + row : row * g.lda + t.k_begin),
+                                              b + (BT ? col * g.ldb + t.k_begin : t.k_begin * g.ldb + col),
+                                              AT ? g.lda : 1, BT ? 1 : g.ldb, t.k_end - t.k_begin);
+        }
     }
 }
 
-__global__ void __launch_bounds__(256)
-splitk_reduce_kernel(const float *__restrict__ partial, GemmArgs g, int batch_count)
+// ---------------------------------------------------------------------------------------------------------------
+// Short kernel: products too small to fill the chip with the tiles above (up to 128 of them; 2048 x 32 x 480: 27 -> 7
+// us, where 16 workgroups of the wide tile take 17).  A workgroup of 8 wavefronts owns 32 rows
+// and 32 TN columns and splits the reduction: wavefront w takes the groups of eight k number w, w + 8, ...  Operands
+// go straight from memory to the fp32 MFMAs (v_mfma_f32_32x32x2_f32: lane half h takes k = 4 h + e of a group in the
+// e-th of its four MFMAs), four groups requested together; the partial tiles meet in LDS, added in order.
+#define GSH_WAVES 8
+
+// k = kg + 4 h .. + 3 of one row or column (elements `step` apart in memory), zeros from k_end on
+template <bool KC>
+__device__ __forceinline__ void gsh_load(const float *__restrict__ p, int64_t step, int64_t kg, int h, int64_t k_end,
+                                         float (&out)[4])
 {
-    const int64_t per = g.rows * g.cols;
-    const int64_t total = per * batch_count;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t bi = i / per, e = i % per;
-        const float *src = partial + bi * g.split_k * per + e;
-        float s = 0.0f;
-        int k = 0;
-        for (; k + 8 <= g.split_k; k += 8) {                        // eight loads in flight, added in order
-            float v[8];
+    const int64_t kq = kg + 4 * h;
+    if (kg + 8 <= k_end) {
+        if (KC) {
+            const floatx4u v = *(const floatx4u *)(p + kq);
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = src[(int64_t)(k + u) * per];
+            for (int e = 0; e < 4; ++e) out[e] = v[e];
+        } else {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) s += v[u];
+            for (int e = 0; e < 4; ++e) out[e] = p[(kq + e) * step];
         }
-        for (; k < g.split_k; ++k) s += src[(int64_t)k * per];
-        g.c[bi * g.stride_c + (e / g.cols) * g.ldc + (e % g.cols)] = s;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const bool in = kq + e < k_end;
+            const float v = p[(in ? kq + e : k_end - 1) * step];
+            out[e] = in ? v : 0.0f;
+        }
     }
+}
+
+template <bool AT, bool BT, int TN>
+__global__ void __launch_bounds__(GSH_WAVES * 64)
+gemm_f32_short_kernel(GemmArgs g, float *__restrict__ partial)
+{
+    constexpr int BN = 32 * TN;
+    constexpr int AHEAD = 4;
+    __shared__ float part[GSH_WAVES][32 * BN];
+    const int lane = pccnn_lane();
+    const int wave = threadIdx.x >> 6;
+    const int r = lane & 31, h = lane >> 5;
+    const GemmTile t = gemm_tile<32, BN>(g);
+    if (!t.valid) return;
+    const int64_t row = t.bm + r < g.rows ? t.bm + r : g.rows - 1;
+    const float *a = g.a + (int64_t)t.batch * g.stride_a + (AT ? row : row * g.lda);
+    const float *b = g.b + (int64_t)t.batch * g.stride_b;
+    const float *bc[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int64_t col = t.bn + 32 * j + r < g.cols ? t.bn + 32 * j + r : g.cols - 1;
+        bc[j] = b + (BT ? col * g.ldb : col);
+    }
+    floatx16 acc[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[j][v] = 0.0f;
+
+    for (int64_t k0 = t.k_begin + wave * 8; k0 < t.k_end; k0 += AHEAD * GSH_WAVES * 8) {
+        float fa[AHEAD][4], fb[AHEAD][TN][4];
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) {
+            const int64_t kg = k0 + q * (GSH_WAVES * 8);            // uniform over the wavefront
+            if (kg >= t.k_end) break;
+            gsh_load<!AT>(a, AT ? g.lda : 1, kg, h, t.k_end, fa[q]);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) gsh_load<BT>(bc[j], BT ? 1 : g.ldb, kg, h, t.k_end, fb[q][j]);
+        }
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) {
+            if (k0 + q * (GSH_WAVES * 8) >= t.k_end) break;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][e], fb[q][j][e], acc[j], 0, 0, 0);
+        }
+    }
+    // register v of lane l: row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32 of the tile
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) part[wave][(8 * (v / 4) + 4 * h + v % 4) * BN + 32 * j + r] = acc[j][v];
+    __syncthreads();
+    int64_t ldc;
+    float *cbase = gemm_output(g, t, partial, ldc);
+    for (int e = threadIdx.x; e < 32 * BN; e += GSH_WAVES * 64) {
+        float s = 0.0f;
+#pragma unroll
+        for (int w = 0; w < GSH_WAVES; ++w) s += part[w][e];
+        const int64_t orow = t.bm + e / BN, ocol = t.bn + e % BN;
+        if (orow < g.rows && ocol < g.cols) cbase[orow * ldc + ocol] = s;
+    }
+}
+
+// Sums the partial products in a fixed order.  LANES threads share an output element (each adds every LANES-th run of
+// splits, eight loads in flight) and meet in LDS: with few elements and many splits one thread's chain of loads would
+// be the whole time.
+template <int LANES>
+__global__ void __launch_bounds__(256)
+splitk_reduce_kernel(const float *__restrict__ partial, float *__restrict__ c, int64_t rows, int64_t cols, int64_t ldc,
+                     int64_t stride_c, int split_k, int batch_count)
+{
+    constexpr int COLS = 256 / LANES;
+    __shared__ float part[LANES][COLS];
+    const int64_t per = rows * cols;
+    const int64_t total = per * batch_count;
+    const int col = threadIdx.x % COLS, lane = threadIdx.x / COLS;
+    const int run = (split_k + LANES - 1) / LANES;
+    const int k0 = lane * run, k1 = k0 + run < split_k ? k0 + run : split_k;
+    for (int64_t base = (int64_t)blockIdx.x * COLS; base < total; base += (int64_t)gridDim.x * COLS) {
+        const int64_t i = base + col;
+        const int64_t bi = i / per, e = i % per;
+        float s = 0.0f;
+        if (i < total) {
+            const float *src = partial + bi * split_k * per + e;
+            int k = k0;
+            for (; k + 8 <= k1; k += 8) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = src[(int64_t)(k + u) * per];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) s += v[u];
+            }
+            for (; k < k1; ++k) s += src[(int64_t)k * per];
+        }
+        if (LANES > 1) {
+            part[lane][col] = s;
+            __syncthreads();
+            if (lane == 0) {
+#pragma unroll
+                for (int l = 1; l < LANES; ++l) s += part[l][col];
+            }
+            __syncthreads();
+        }
+        if (lane == 0 && i < total) c[bi * stride_c + (e / cols) * ldc + (e % cols)] = s;
+    }
+}
+
+int pccnn_splitk_reduce(const float *partial, float *c, int64_t rows, int64_t cols, int64_t ldc, int64_t stride_c,
+                        int split_k, int batch, hipStream_t s)
+{
+    const int64_t total = rows * cols * batch;
+    // one thread per element when that fills the chip
+    const int lanes = total >= (1 << 17) || split_k <= 8 ? 1 : 8;
+    int64_t blocks = pccnn_ceil_div(total * lanes, 256);
+    if (blocks > 4096) blocks = 4096;
+    if (lanes == 1)
+        splitk_reduce_kernel<1><<<(unsigned)blocks, 256, 0, s>>>(partial, c, rows, cols, ldc, stride_c, split_k, batch);
+    else
+        splitk_reduce_kernel<8><<<(unsigned)blocks, 256, 0, s>>>(partial, c, rows, cols, ldc, stride_c, split_k, batch);
+    PCCNN_LAUNCH_CHECK();
+    return PCCNN_OK;
+}
+
+// Which tile a product takes: (rows, columns) of a workgroup's tile; `is_short`: the short kernel.
+struct GemmPlan {
+    int bm, bn;
+    bool is_short;
+};
+
+static int64_t gemm_tiles(int64_t rows, int64_t cols, int bm, int bn)
+{
+    return pccnn_ceil_div(rows, bm) * pccnn_ceil_div(cols, bn);
+}
+
+// `copies`: how many times the tiles of one product are in the launch (batch x split).
+static GemmPlan gemm_plan(int64_t rows, int64_t cols, int64_t copies, int64_t lda, int64_t ldb)
+{
+    // the wide tile that pads the columns least, weighted with what a column costs in it (65 536 x 256 x 1920: 352 us
+    // with 128 columns, 392 with 64)
+    GemmPlan p = {128, 128, false};
+    if (cols <= 32) p.bn = 32;
+    else if (cols <= 64) p.bn = 64;
+    else {
+        const double c128 = 1.0 * pccnn_ceil_div(cols, 128) * 128, c96 = 1.08 * pccnn_ceil_div(cols, 96) * 96,
+                     c64 = 1.12 * pccnn_ceil_div(cols, 64) * 64;
+        p.bn = c128 <= c96 && c128 <= c64 ? 128 : (c96 <= c64 ? 96 : 64);
+    }
+    // nearly two workgroups per CU (of the 96-column tile one) or the 64 x 64 tile: 14 065 x 64 x 512 20 us with 110
+    // workgroups of 128 x 64, 16 with 220; 12 000 x 250 x 200 17.7 with 376, 16.1 with 752; 37 675 x 96 x 720 51 with
+    // 295 workgroups of 128 x 96, 56 with 1178
+    if (p.bn > 32 && gemm_tiles(rows, cols, 128, p.bn) * copies < (p.bn == 96 ? 256 : 448)) p.bm = p.bn = 64;
+    if (gemm_tiles(rows, cols, p.bm, p.bn) * copies <= 128 || lda >= (1ll << 22) || ldb >= (1ll << 22)) {
+        p.is_short = true;
+        p.bm = 32;
+        p.bn = cols > 32 && gemm_tiles(rows, cols, 32, 64) * copies > 256 ? 64 : 32;
+    }
+    return p;
+}
+
+// A split of the reduction for a product whose output has few tiles (d_weights = P^T x dOut): two workgroups per CU of
+// the wide tile with 512 or more of the reduction each, else of the 64 x 64 tile with 128 or more.  What
+// the split writes and the last kernel reads again is bounded by the workspace.
+int pccnn_gemm_f32_split(int64_t rows, int64_t cols, int64_t inner, int batch, size_t workspace_floats)
+{
+    if (inner < 512 || rows < 1 || cols < 1) return 1;
+    const int64_t room = (int64_t)(workspace_floats / ((size_t)rows * cols * batch));
+    const int64_t most = room < 512 ? room : 512;
+    const GemmPlan wide = gemm_plan(rows, cols, 1 << 20, 1, 1);
+    // (not more than two per CU: 540 workgroups of 1920 x 256 x 65 536 take 485 us, 510 take 386)
+    int64_t split = 512 / (gemm_tiles(rows, cols, 128, wide.bn) * batch);
+    if (split < 1) split = 1;
+    if (split > most || inner / split < 512) {
+        split = 512 / (gemm_tiles(rows, cols, wide.bn > 32 ? 64 : 128, wide.bn > 32 ? 64 : 32) * batch);
+        if (split > inner / 128) split = inner / 128;
+        if (split > most) split = most;
+    }
+    return split < 1 ? 1 : (int)split;
 }
 
 extern "C" int pccnn_gemm_f32(const float *a, const float *b, float *c, int64_t rows, int64_t cols, int64_t inner,
@@ -509,19 +633,17 @@ extern "C" int pccnn_gemm_f32(const float *a, const float *b, float *c, int64_t 
                   "pccnn_gemm_f32: leading dimension too small (lda=%lld ldb=%lld ldc=%lld)", (long long)lda,
                   (long long)ldb, (long long)ldc);
     if (split_k < 1) split_k = 1;
+    GemmPlan plan = gemm_plan(rows, cols, (int64_t)batch * split_k, lda, ldb);
     GemmArgs g;
     g.a = a; g.b = b; g.c = c;
     g.rows = rows; g.cols = cols; g.inner = inner;
     g.lda = lda; g.ldb = ldb; g.ldc = ldc;
     g.stride_a = stride_a; g.stride_b = stride_b; g.stride_c = stride_c;
-    int64_t chunk = pccnn_ceil_div(pccnn_ceil_div(inner > 0 ? inner : 1, split_k), GT_K) * GT_K;
+    const int unit = plan.is_short ? GSH_WAVES * 8 : GS_K;
+    const int64_t chunk = pccnn_ceil_div(pccnn_ceil_div(inner > 0 ? inner : 1, split_k), unit) * unit;
     split_k = (int)pccnn_ceil_div(inner > 0 ? inner : 1, chunk);
     g.split_k = split_k;
     g.k_chunk = chunk;
-    g.aligned = ((uintptr_t)a % 16 == 0) && ((uintptr_t)b % 16 == 0) && (lda % 4 == 0) && (ldb % 4 == 0) &&
-                (stride_a % 4 == 0) && (stride_b % 4 == 0);
-    // units run along the reduction index where that is contiguous in memory, else along the rows / columns
-    g.whole_units = g.aligned && ((a_trans ? rows : inner) % 4 == 0) && ((b_trans ? inner : cols) % 4 == 0);
     float *partial = nullptr;
     if (split_k > 1) {
         size_t need = (size_t)batch * split_k * rows * cols * sizeof(float);
@@ -530,51 +652,37 @@ extern "C" int pccnn_gemm_f32(const float *a, const float *b, float *c, int64_t 
         partial = (float *)workspace;
     }
     hipStream_t s = (hipStream_t)stream;
-    // The kernel for full tiles takes every shape that has them, except products with fewer than 12 k tiles per
-    // workgroup: there the prologue and the epilogue weigh more than the loop, and the general kernel, which
-    // keeps four instead of three waves per SIMD, is ahead (65 536 x 1024 x 128, B transposed: 162 against 166 us).
-    // Lane offsets inside a tile are 32-bit byte offsets: 256 rows of the leading dimension must fit.
-    const bool full_128 = rows % 128 == 0, full_64 = rows % 64 == 0;
-    const bool full_ok = g.aligned && cols % GT_N == 0 && inner % GT_K == 0 && chunk >= 12 * GT_K && lda < (1ll << 20) &&
-                         ldb < (1ll << 20) &&
-                         (split_k > 1 ? (uintptr_t)partial % 16 == 0
-                                      : ldc % 4 == 0 && (uintptr_t)c % 16 == 0 && stride_c % 4 == 0);
-    // 128-row tiles unless that leaves the chip short of workgroups: the general kernel wants about four per CU,
-    // the kernel for full tiles is ahead with 128-row tiles from one per CU on (65 536 x 128 x 1024: 140 against
-    // 153 us with 64-row tiles; the wider tile needs fewer load instructions per MFMA)
-    const int64_t wg128 = pccnn_ceil_div(cols, GT_N) * pccnn_ceil_div(rows, 128) * batch * split_k;
-    int bm_tile = wg128 >= 1024 ? 128 : 64;
-    bool full_tiles = false;
-    if (full_ok && full_128 && wg128 >= 256) { bm_tile = 128; full_tiles = true; }
-    else if (full_ok && full_64 && bm_tile == 64) full_tiles = true;
-    g.tiles_x = (int)pccnn_ceil_div(cols, GT_N);
-    g.tiles_y = (int)pccnn_ceil_div(rows, bm_tile);
+    g.tiles_x = (int)pccnn_ceil_div(cols, plan.bn);
+    g.tiles_y = (int)pccnn_ceil_div(rows, plan.bm);
     g.total_wg = (int64_t)g.tiles_x * g.tiles_y * batch * split_k;
     PCCNN_REQUIRE(g.total_wg < (1ll << 31) - GEMM_XCDS, PCCNN_ERR_UNSUPPORTED, "pccnn_gemm_f32: grid too large");
     dim3 grid((unsigned)(pccnn_ceil_div(g.total_wg, GEMM_XCDS) * GEMM_XCDS));
     {
         PccnnTimed timed(PCCNN_T_GEMM, s);
-#define GEMM_GO(AT, BT)                                                                       \
-    do {                                                                                      \
-        if (full_tiles) {                                                                     \
-            if (bm_tile == 128) gemm_f32_full_tiles_kernel<AT, BT, 128><<<grid, 256, 0, s>>>(g, partial); \
-            else gemm_f32_full_tiles_kernel<AT, BT, 64><<<grid, 256, 0, s>>>(g, partial);     \
-        } else if (bm_tile == 128) gemm_f32_mfma_kernel<AT, BT, 128><<<grid, 256, 0, s>>>(g, partial); \
-        else gemm_f32_mfma_kernel<AT, BT, 64><<<grid, 256, 0, s>>>(g, partial);                 \
+#define SPLIT_GO(AT, BT, WM, WN, TM, TN)                                                                          \
+    do {                                                                                                          \
+        if (chunk > GS_ONE_SUM) gemm_f32_split_kernel<AT, BT, WM, WN, TM, TN, true><<<grid, 256, 0, s>>>(g, partial); \
+        else gemm_f32_split_kernel<AT, BT, WM, WN, TM, TN, false><<<grid, 256, 0, s>>>(g, partial);                 \
+    } while (0)
+#define GEMM_GO(AT, BT)                                                                                           \
+    do {                                                                                                          \
+        if (plan.is_short) {                                                                                      \
+            if (plan.bn == 64) gemm_f32_short_kernel<AT, BT, 2><<<grid, GSH_WAVES * 64, 0, s>>>(g, partial);      \
+            else gemm_f32_short_kernel<AT, BT, 1><<<grid, GSH_WAVES * 64, 0, s>>>(g, partial);                    \
+        } else if (plan.bm == 64) SPLIT_GO(AT, BT, 2, 2, 1, 1);                                                   \
+        else if (plan.bn == 128) SPLIT_GO(AT, BT, 2, 2, 2, 2);                                                    \
+        else if (plan.bn == 96) SPLIT_GO(AT, BT, 4, 1, 1, 3);                                                     \
+        else if (plan.bn == 64) SPLIT_GO(AT, BT, 2, 2, 2, 1);                                                     \
+        else SPLIT_GO(AT, BT, 4, 1, 1, 1);                                                                        \
     } while (0)
         if (!a_trans && !b_trans) GEMM_GO(false, false);
         else if (!a_trans && b_trans) GEMM_GO(false, true);
         else if (a_trans && !b_trans) GEMM_GO(true, false);
         else GEMM_GO(true, true);
 #undef GEMM_GO
+#undef SPLIT_GO
     }
     PCCNN_LAUNCH_CHECK();
-    if (split_k > 1) {
-        int64_t total = rows * cols * batch;
-        int64_t blocks = pccnn_ceil_div(total, 256);
-        if (blocks > 4096) blocks = 4096;
-        splitk_reduce_kernel<<<(unsigned)blocks, 256, 0, s>>>(partial, g, batch);
-        PCCNN_LAUNCH_CHECK();
-    }
+    if (split_k > 1) return pccnn_splitk_reduce(partial, c, rows, cols, ldc, stride_c, split_k, batch, s);
     return PCCNN_OK;
 }

@@ -249,28 +249,6 @@ gemm_bf16_mfma_kernel(GemmBf16Args g, float *__restrict__ partial)
         }
 }
 
-__global__ void __launch_bounds__(256)
-bg_splitk_reduce_kernel(const float *__restrict__ partial, GemmBf16Args g, int batch_count)
-{
-    const int64_t per = g.rows * g.cols;
-    const int64_t total = per * batch_count;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t bi = i / per, e = i % per;
-        const float *src = partial + bi * g.split_k * per + e;
-        float s = 0.0f;
-        int k = 0;
-        for (; k + 8 <= g.split_k; k += 8) {                        // eight loads in flight, added in order
-            float v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = src[(int64_t)(k + u) * per];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) s += v[u];
-        }
-        for (; k < g.split_k; ++k) s += src[(int64_t)k * per];
-        g.c[bi * g.stride_c + (e / g.cols) * g.ldc + (e % g.cols)] = s;
-    }
-}
-
 // fp32 -> bf16, round to nearest even (NaN stays NaN).
 __global__ void __launch_bounds__(256)
 f32_to_bf16_kernel(const float *__restrict__ src, uint16_t *__restrict__ dst, int64_t count)
@@ -348,12 +326,6 @@ extern "C" int pccnn_gemm_bf16(const uint16_t *a, const uint16_t *b, float *c, i
 #undef GEMM_GO
     }
     PCCNN_LAUNCH_CHECK();
-    if (split_k > 1) {
-        int64_t total = rows * cols * batch;
-        int64_t blocks = pccnn_ceil_div(total, 256);
-        if (blocks > 4096) blocks = 4096;
-        bg_splitk_reduce_kernel<<<(unsigned)blocks, 256, 0, s>>>(partial, g, batch);
-        PCCNN_LAUNCH_CHECK();
-    }
+    if (split_k > 1) return pccnn_splitk_reduce(partial, c, rows, cols, ldc, stride_c, split_k, batch, s);
     return PCCNN_OK;
 }

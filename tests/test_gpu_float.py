@@ -54,6 +54,77 @@ def test_gemm_against_float64(rows, cols, inner, at, bt, split):
     assert relerr(tc.cpu().numpy(), exp) < 1e-5
 
 
+def _gemm_f32(a, b, at, bt, split=1):
+    from pccnn_lib_amd import _lib
+    rows, inner = (a.shape[1], a.shape[0]) if at else a.shape
+    cols = b.shape[0] if bt else b.shape[1]
+    ta, tb = t(a), t(b)
+    tc = torch.full((rows, cols), float("nan"), dtype=torch.float32, device=DEV)
+    ws = torch.empty(split * rows * cols * 4 + 256, dtype=torch.uint8, device=DEV)
+    _lib.call("pccnn_gemm_f32", _lib.P(ta.data_ptr()), _lib.P(tb.data_ptr()), _lib.P(tc.data_ptr()), rows, cols, inner,
+              at, bt, a.shape[1], b.shape[1], cols, 1, 0, 0, 0, split, _lib.P(ws.data_ptr()), ws.numel(),
+              _lib.P(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    return tc.cpu().numpy()
+
+
+# every tile of the split kernel (128 x 128, 96, 64 and 32; 64 x 64) in the three layouts of the convolutions, with
+# odd leading dimensions, row / column / reduction remainders, one and two sums per element; and the short kernel
+@pytest.mark.parametrize("rows,cols,inner", [
+    (60001, 129, 65), (57345, 128, 1056), (33333, 95, 67), (30011, 96, 1057), (58001, 63, 33), (57345, 64, 1088),
+    (20001, 31, 1), (16385, 32, 1100), (9001, 127, 31), (9001, 33, 1090), (33, 65, 64), (31, 1, 513), (1, 200, 9)])
+@pytest.mark.parametrize("at,bt", [(0, 0), (0, 1), (1, 0)])
+def test_gemm_is_as_precise_as_fp32_arithmetic(rows, cols, inner, at, bt):
+    # bound: fp32 sums of `inner` products, one rounding (2^-24) per product and per addition, errors adding up like a
+    # random walk of sqrt(inner) steps over partial sums that grow like sqrt(k): sqrt(inner / 2 + 1) 2^-24 relative to
+    # the result's norm
+    rng = np.random.default_rng(rows + cols + inner)
+    a = rng.normal(size=(inner, rows) if at else (rows, inner)).astype(np.float32)
+    b = rng.normal(size=(cols, inner) if bt else (inner, cols)).astype(np.float32)
+    exp = (a.T if at else a).astype(np.float64) @ (b.T if bt else b).astype(np.float64)
+    got = _gemm_f32(a, b, at, bt)
+    assert np.linalg.norm(got - exp) / np.linalg.norm(exp) < np.sqrt(inner / 2 + 1) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("rows,cols,inner,split", [(200, 40, 3000, 23), (24, 33, 7327, 57), (600, 130, 1000, 3)])
+def test_gemm_split_reduction_with_many_partial_products(rows, cols, inner, split):
+    rng = np.random.default_rng(rows)
+    a, b = (rng.normal(size=(inner, n)).astype(np.float32) for n in (rows, cols))
+    exp = a.T.astype(np.float64) @ b.astype(np.float64)
+    assert relerr(_gemm_f32(a, b, 1, 0, split), exp) < 1e-5
+
+
+def test_gemm_of_huge_tiny_and_non_finite_values():
+    # 65 536 rows: the split kernel.  Values that round up to infinity as bf16, infinities and NaNs give what fp32
+    # arithmetic gives, in the rows they stand in; rows of very small values keep fp32's relative precision.
+    rng = np.random.default_rng(4)
+    a = rng.normal(size=(65536, 96)).astype(np.float32)
+    b = rng.normal(size=(96, 128)).astype(np.float32)
+    b[np.abs(b) < 0.1] = 0.5
+    a[5, 3] = np.inf
+    a[700, 90] = -np.inf
+    a[1300, 17] = np.nan
+    a[9000, :] = 0.0
+    a[9000, 40] = 3.4028e38
+    b[40, :] *= 0.25
+    a[20000:20100] *= 1e-37
+    with np.errstate(all="ignore"):
+        exp = a.astype(np.float64) @ b.astype(np.float64)
+    got = _gemm_f32(a, b, 0, 0)
+    for row in (5, 700, 1300):
+        assert np.array_equal(np.isnan(got[row]), np.isnan(exp[row]))
+        assert np.array_equal(got[row][~np.isnan(exp[row])], exp[row][~np.isnan(exp[row])].astype(np.float32))
+    with np.errstate(over="ignore"):
+        big = exp[9000].astype(np.float32)
+    assert np.array_equal(np.isinf(got[9000]), np.isinf(big))
+    fine = np.isfinite(big)
+    assert fine.any() and np.allclose(got[9000][fine], big[fine], rtol=1e-6)
+    # (single results of the tiny rows are subnormal: absolute steps of 2^-149, 1e-8 of the largest)
+    assert relerr(got[20000:20100] * 2.0 ** 100, exp[20000:20100] * 2.0 ** 100) < 1e-5
+    rest = np.setdiff1d(np.arange(65536), [5, 700, 1300, 9000])
+    assert relerr(got[rest], exp[rest]) < 1e-5
+
+
 @pytest.mark.parametrize("m,mlps,inner,co", [(200, 2, 48, 24), (256, 2, 208, 128), (32768, 3, 192, 128)])
 def test_gemm_batched_strided(m, mlps, inner, co):
     # the second and third shapes have full tiles: the kernel without bounds checks, 64-row and 128-row tiles
