@@ -175,6 +175,138 @@ conv_proj_fwd_kernel(ConvGeom g, const float *__restrict__ feats, void *__restri
     }
 }
 
+// Forward projection of at most 16 basis values on the matrix cores: P[k][f] = sum over the pairs of w[k][t] F[t][f] is
+// a product per sample with the pairs as its inner dimension, four of them per v_mfma_f32_16x16x4_f32.  One wavefront
+// per (sample, 64 features), lane = (q = lane / 16, c = lane % 16): it evaluates basis value c of pair 4 i + q and
+// loads feature 16 u + c of that pair's row, which are the operands as the instruction takes them; no value passes
+// through LDS but the pairs' geometry.  Products and sums are fp32 as on the vector ALU.
+// conv_proj_fwd_kernel, which takes 17 and more basis values, is bound by its broadcast reads of the basis values from
+// LDS and by the vector ALU; at 16 and fewer it was the slower one at every size measured, us there / here: 65 536
+// samples, 14.4 pairs, 64 features x 16: 89 / 81, bf16 out 84 / 72; 65 536, 18.1, 128 x 15: 235 / 186; 37 675, 21.5,
+// 48 x 15: 73 / 55; 120 000, 13.5, 128 x 15: 355 / 319 (the write of 922 MB).  What bounds it now is that write.
+template <int BASIS, int KPAD, bool BF16>
+__global__ void __launch_bounds__(64)
+conv_proj_fwd_mfma_kernel(ConvGeom g, const float *__restrict__ feats, void *__restrict__ proj_out)
+{
+    static_assert(KPAD == 8 || KPAD == 16, "one 16-row tile of basis values");
+    constexpr bool GEOM = BASIS != BASIS_EXPLICIT;      // explicit basis values need no positions
+    constexpr int STEPS = 2;                            // groups of four pairs in flight
+    __shared__ float4 geo_lds[GEOM ? 64 : 1];           // (offset, density) of the chunk's pairs
+    __shared__ int nidx_lds[64];                        // and their points
+    __shared__ __attribute__((aligned(16))) float tile[64 * KPAD];
+    const int lane = threadIdx.x, q = lane / 16, c = lane % 16;
+    const int64_t s = conv_sample_of_block(blockIdx.x, g.m);
+    if (s >= g.m) return;                               // (the grid is padded to a multiple of the XCD count)
+    const int f0 = blockIdx.y * 64;
+    const int nf = (g.c_in - f0) < 64 ? (g.c_in - f0) : 64;
+    const int lo = s > 0 ? g.ends[s - 1] : 0;
+    const int hi = g.ends[s];
+    float sx = 0.f, sy = 0.f, sz = 0.f, ir0 = 1.f, ir1 = 1.f, ir2 = 1.f;
+    if (GEOM) {
+        sx = g.samples[s * 3 + 0]; sy = g.samples[s * 3 + 1]; sz = g.samples[s * 3 + 2];
+        ir0 = 1.0f / g.radii[0]; ir1 = 1.0f / g.radii[1]; ir2 = 1.0f / g.radii[2];
+    }
+    LaneBasis<BASIS> lb;
+    lb.load(g, c);
+
+    floatx4_t acc[4];                                   // acc[u][r]: basis value 4 q + r, feature 16 u + c
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc[u] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+
+    for (int cb = lo; cb < hi; cb += 64) {
+        const int cnt = (hi - cb) < 64 ? (hi - cb) : 64;
+        int nidx = 0;
+        if (lane < cnt) nidx = g.neigh[cb + lane].x;
+        nidx_lds[lane] = nidx;
+        __syncthreads();
+        // Features of the pairs j0 + 4 i + q (zeros past the chunk's end).
+        auto load_rows = [&](int j0, float (&row)[STEPS][4]) {
+#pragma unroll
+            for (int i = 0; i < STEPS; ++i) {
+                const int j = j0 + 4 * i + q;           // < 64: j0 is a multiple of 8 below cnt
+                const float *src = feats + (int64_t)nidx_lds[j] * g.c_in + f0 + c;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) row[i][u] = (j < cnt && 16 * u + c < nf) ? src[16 * u] : 0.0f;
+            }
+        };
+        float row[STEPS][4];
+        load_rows(0, row);
+        if (GEOM) {
+            float4 ge = make_float4(0.f, 0.f, 0.f, 1.f);
+            if (lane < cnt) {
+                ge.x = (g.pts[(int64_t)nidx * 3 + 0] - sx) * ir0;
+                ge.y = (g.pts[(int64_t)nidx * 3 + 1] - sy) * ir1;
+                ge.z = (g.pts[(int64_t)nidx * 3 + 2] - sz) * ir2;
+                if (BasisTraits<BASIS>::uses_pdf) ge.w = g.pdf[nidx];
+            }
+            geo_lds[lane] = ge;
+            __syncthreads();
+        }
+        for (int j0 = 0; j0 < cnt; j0 += 4 * STEPS) {
+            float row_next[STEPS][4];
+            const bool more = j0 + 4 * STEPS < cnt;                 // uniform
+            if (more) load_rows(j0 + 4 * STEPS, row_next);
+#pragma unroll
+            for (int i = 0; i < STEPS; ++i) {
+                const int j = j0 + 4 * i + q;
+                float4 ge = make_float4(0.f, 0.f, 0.f, 1.f);
+                if (GEOM) ge = geo_lds[j];
+                const float w = (j < cnt) ? pair_basis<BASIS>(g, lb, (int64_t)cb + j, ge.x, ge.y, ge.z, ge.w) : 0.0f;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, row[i][u], acc[u], 0, 0, 0);
+            }
+            if (more) {
+#pragma unroll
+                for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) row[i][u] = row_next[i][u];
+            }
+        }
+        __syncthreads();
+    }
+    const int64_t dst_at = ((int64_t)s * g.c_in + f0) * g.k;
+    if (g.k == KPAD) {
+        // four neighboring basis values per lane: every store instruction writes one contiguous run
+        if (4 * q >= KPAD) return;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int f = 16 * u + c;
+            if (f >= nf) continue;
+            if (BF16) {
+                // the projection leaves as bf16 (round to nearest even): the operand format of the bf16 contraction
+                uint2 o;
+                o.x = pccnn_bf16_bits(acc[u][0]) | ((uint32_t)pccnn_bf16_bits(acc[u][1]) << 16);
+                o.y = pccnn_bf16_bits(acc[u][2]) | ((uint32_t)pccnn_bf16_bits(acc[u][3]) << 16);
+                *(uint2 *)((uint16_t *)proj_out + dst_at + f * KPAD + 4 * q) = o;
+            } else {
+                // whole lines that nothing reads before the next kernel: stored past the L2 (not the bf16 ones: half
+                // the size, much of them is still in cache when the contraction reads them)
+                __builtin_nontemporal_store(acc[u], (floatx4_t *)((float *)proj_out + dst_at + f * KPAD + 4 * q));
+            }
+        }
+        return;
+    }
+    // Rows that are no multiple of four values are packed in LDS first, for the same contiguous stores.
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (4 * q + r < g.k) tile[(16 * u + c) * g.k + 4 * q + r] = acc[u][r];
+    __syncthreads();
+    const int total = nf * g.k;
+    if (BF16) {
+        uint16_t *dst = (uint16_t *)proj_out + dst_at;
+        for (int i = lane; i < total; i += 64) dst[i] = pccnn_bf16_bits(tile[i]);
+    } else {
+        float *dst = (float *)proj_out + dst_at;
+        if (((uintptr_t)dst & 15) == 0 && (total & 3) == 0) {
+            for (int i = lane; i < total / 4; i += 64) ((float4 *)dst)[i] = ((const float4 *)tile)[i];
+        } else {
+            for (int i = lane; i < total; i += 64) dst[i] = tile[i];
+        }
+    }
+}
+
 // Forward projection for at most 32 input features.  With lane = feature, most of a wavefront would idle; here
 // G = 64 / FPAD pairs are processed side by side, lane = (pair slot, feature): every lane keeps K partial sums for
 // its feature over the pairs that fall into its slot, and the slots are added at the end (DPP rotations and row
@@ -1184,13 +1316,19 @@ static int launch_proj_fwd(const ConvGeom &g, const float *feats, void *proj, hi
         if (bf16) conv_proj_fwd_kernel<BASIS, KP, true><<<grid, 64, 0, s>>>(g, feats, proj);  \
         else conv_proj_fwd_kernel<BASIS, KP, false><<<grid, 64, 0, s>>>(g, feats, proj);      \
     } while (0)
+#define MFMA_GO(KP)                                                                              \
+    do {                                                                                         \
+        if (bf16) conv_proj_fwd_mfma_kernel<BASIS, KP, true><<<grid, 64, 0, s>>>(g, feats, proj);  \
+        else conv_proj_fwd_mfma_kernel<BASIS, KP, false><<<grid, 64, 0, s>>>(g, feats, proj);      \
+    } while (0)
     switch (kpad_of(g.k)) {
-    case 8: PROJ_GO(8); break;
-    case 16: PROJ_GO(16); break;
+    case 8: MFMA_GO(8); break;
+    case 16: MFMA_GO(16); break;
     case 32: PROJ_GO(32); break;
     default: PROJ_GO(64); break;
     }
 #undef PROJ_GO
+#undef MFMA_GO
     PCCNN_LAUNCH_CHECK();
     return PCCNN_OK;
 }

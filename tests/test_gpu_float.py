@@ -249,6 +249,35 @@ def test_kpconv_forward_and_grads(ops, oracle, k, c_in, c_out, distinct):
         assert mixed_close(got.cpu().numpy(), e), name
 
 
+@pytest.mark.parametrize("k", [5, 8, 9, 15, 16, 17])
+@pytest.mark.parametrize("c_in", [33, 64, 65, 130])
+def test_forward_projection_at_the_edges_of_its_tiles(ops, oracle, k, c_in):
+    """Pair counts around the groups of four, eight and 64 that a projection kernel takes at a time (none at all among
+    them), feature counts around its blocks of 64 and tiles of 16, basis counts around its tiles of 8 and 16."""
+    rng = np.random.default_rng(1000 * k + c_in)
+    counts = [0, 1, 3, 4, 5, 7, 8, 9, 0, 31, 63, 64, 65, 72, 73, 130, 2]
+    pts = rng.uniform(0.0, 0.2, (140, 3)).astype(np.float32)
+    smp = rng.uniform(0.0, 0.2, (len(counts), 3)).astype(np.float32)
+    neigh = np.concatenate([np.stack([rng.permutation(140)[:n], np.full(n, i)], 1)
+                            for i, n in enumerate(counts)]).astype(np.int32)
+    ends = np.cumsum(counts).astype(np.int32)
+    radii = np.full(3, 0.2, np.float32)
+    kp, sigma = synthetic.kernel_points_sphere(1, k)
+    feats = rng.normal(size=(140, c_in)).astype(np.float32)
+    w = rng.normal(0, np.sqrt(1.0 / (k * c_in)), (k * c_in, 24)).astype(np.float32)
+    exp = oracle.kpconv(pts, feats, smp, neigh, ends, radii, kp, sigma, w)
+    out = ops.kp_conv(t(pts), t(feats), t(smp), t(neigh), t(ends), t(radii), t(kp), sigma, t(w)).cpu().numpy()
+    # sums of at most 130 pairs and 2210 products in fp32
+    assert relerr(out, exp) < FWD_TOL
+    assert mixed_close(out, exp)
+    assert np.all(out[[0, 8]] == 0.0)
+    # an infinity stays with the samples that have its point among their neighbors
+    feats[neigh[-1, 0], c_in - 1] = np.inf
+    hit = np.array([np.any(neigh[neigh[:, 1] == i, 0] == neigh[-1, 0]) for i in range(len(counts))])
+    again = ops.kp_conv(t(pts), t(feats), t(smp), t(neigh), t(ends), t(radii), t(kp), sigma, t(w)).cpu().numpy()
+    assert np.array_equal(again[~hit], out[~hit])
+
+
 @pytest.mark.parametrize("hidden,mlps,c_in,c_out,distinct", [(16, 1, 64, 128, False), (8, 2, 32, 24, True),
                                                              (16, 1, 3, 16, True), (4, 4, 8, 8, False)])
 def test_mcconv_forward_and_grads(ops, oracle, hidden, mlps, c_in, c_out, distinct):
