@@ -516,6 +516,7 @@ conv_proj_bwd_kernel(ConvGeom g, const float *__restrict__ feats, const float *_
     LaneBasis<BASIS> lb;
     lb.load(g, k);
     const int fblocks = (g.c_in + 63) / 64;
+    if (want_df) feat_grads += (int64_t)(blockIdx.x % PCCNN_XCDS) * g.feat_copy_stride;
     // gradients towards positions or densities wanted (uniform): otherwise the per-pair sums over the basis index
     // and their hand-over through LDS are skipped
     const bool geometry = d_pts != nullptr || d_samples != nullptr || d_pdf != nullptr || pair_grads != nullptr;
@@ -1026,6 +1027,31 @@ conv_rows_gather_kernel(const float *__restrict__ rows, const int32_t *__restric
         }
         for (; j < hi; ++j) acc += rows[(int64_t)index[j] * c_in + f];
         d_feats[n * c_in + f] = acc;
+    }
+}
+
+// Sum of the XCDs' copies of the feature gradients, in the order of the copies: one thread per four floats, the eight
+// reads in flight together.
+__global__ void __launch_bounds__(256)
+conv_copies_sum_kernel(const float *__restrict__ copies, int64_t stride, int64_t count, float *__restrict__ out)
+{
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= count) return;
+    float4 v[PCCNN_XCDS];
+#pragma unroll
+    for (int x = 0; x < PCCNN_XCDS; ++x) v[x] = *(const float4 *)(copies + x * stride + i);
+    float4 sum = v[0];
+#pragma unroll
+    for (int x = 1; x < PCCNN_XCDS; ++x) {
+        sum.x += v[x].x; sum.y += v[x].y; sum.z += v[x].z; sum.w += v[x].w;
+    }
+    if (i + 4 <= count && (((uintptr_t)(out + i)) & 15) == 0) {
+        *(float4 *)(out + i) = sum;
+    } else {
+        const float tail[4] = {sum.x, sum.y, sum.z, sum.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (i + e < count) out[i + e] = tail[e];
     }
 }
 
@@ -1598,6 +1624,15 @@ static int conv_backward(ConvGeom g, const float *feats, const float *weights, c
                            workspace_bytes >= pccnn_conv_workspace_bytes_deterministic(g.n, g.m, g.t, g.c_in, g.k, c_out);
     const bool rows_route = det || rows_auto;
     g.deterministic = rows_route ? 1 : 0;
+    // Few points with many pairs each (the way back up a hierarchy): the atomics of the whole chip meet in a small
+    // array.  One copy of it per XCD, added up afterwards, in the buffer of the projection, which is free by then:
+    // 4800 points, 1.62 M pairs (337 to a point), 128 features: 815 -> 710 us, the sum 5 us.  With 14 pairs to a point
+    // and 16.8 MB of gradients the kernel gains nothing (255 us either way) and clearing and adding the copies costs
+    // 40 us; from 64 pairs to a point on, that cost is below a tenth of the atomics' own.
+    const int64_t copy_stride = (g.n * g.c_in + 3) / 4 * 4;
+    const bool copies = !rows_route && want_f && g.c_in > 32 && g.m > 0 && g.t / 64 >= g.n &&
+                        copy_stride <= g.m * g.c_in * g.k / PCCNN_XCDS;
+    g.feat_copy_stride = copies ? copy_stride : 0;
     PccnnArena arena(workspace, workspace_bytes);
     const int64_t partial_rows = det ? g.m : PARAM_ROWS;
     const int reduce_groups = det ? PARAM_REDUCE_GROUPS_PER_SAMPLE : PARAM_REDUCE_GROUPS;
@@ -1611,7 +1646,7 @@ static int conv_backward(ConvGeom g, const float *feats, const float *weights, c
     const bool gather = (mirror != nullptr || det) && Tr::differentiable && (want_pts || want_pdf) && g.m > 0 && g.t > 0;
     // the accumulators to clear; the launch follows below, together with the bf16 copies
     ConvPrepJobs prep = {};
-    if (want_f && !rows_route) { prep.zero[0] = d_feats; prep.zero_count[0] = g.n * g.c_in; }
+    if (want_f && !rows_route && !copies) { prep.zero[0] = d_feats; prep.zero_count[0] = g.n * g.c_in; }
     if (want_pts && !gather) { prep.zero[1] = d_pts; prep.zero_count[1] = g.n * 3; }
     if (want_pdf && !gather) { prep.zero[2] = d_pdf; prep.zero_count[2] = g.n; }
     if (g.m == 0 || g.t == 0) {
@@ -1697,10 +1732,16 @@ static int conv_backward(ConvGeom g, const float *feats, const float *weights, c
                             co, inner * co, inner, 1, nullptr, 0, s);
     }
     if (rc != PCCNN_OK) return rc;
+    if (copies) {
+        // the weights' gradient was the last to read the projection
+        ConvPrepJobs clear = {};
+        clear.zero[0] = proj_ws; clear.zero_count[0] = copy_stride * PCCNN_XCDS;
+        if ((rc = conv_prep(clear, s)) != PCCNN_OK) return rc;
+    }
     BasisGradOut o = {basis_g, want_pts ? d_pts : nullptr, want_pts ? d_samples : nullptr, want_pdf ? d_pdf : nullptr,
                       (want_par && Tr::differentiable) ? partials : nullptr, gather ? pair_grads : nullptr};
-    if ((rc = launch_proj_bwd<BASIS>(g, feats, d_proj, want_f ? (rows_route ? df_rows : d_feats) : nullptr, want_basis, o,
-                                     s)) != PCCNN_OK)
+    if ((rc = launch_proj_bwd<BASIS>(g, feats, d_proj, want_f ? (rows_route ? df_rows : copies ? proj_ws : d_feats) : nullptr,
+                                     want_basis, o, s)) != PCCNN_OK)
         return rc;
     if (rows_route && want_f) {
         const int lanes = g.c_in <= 8 ? 8 : (g.c_in <= 16 ? 16 : (g.c_in <= 32 ? 32 : 64));
@@ -1712,6 +1753,11 @@ static int conv_backward(ConvGeom g, const float *feats, const float *weights, c
         else if (lanes == 32) ROWS_GO(32);
         else ROWS_GO(64);
 #undef ROWS_GO
+        PCCNN_LAUNCH_CHECK();
+    }
+    if (copies) {
+        conv_copies_sum_kernel<<<(unsigned)pccnn_ceil_div(copy_stride / 4, 256), 256, 0, s>>>(proj_ws, copy_stride,
+                                                                                             g.n * g.c_in, d_feats);
         PCCNN_LAUNCH_CHECK();
     }
     if (gather) {

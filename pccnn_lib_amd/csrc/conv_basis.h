@@ -41,6 +41,8 @@ struct ConvGeom {
     // Backward pass without float atomics: the feature-gradient row of a pair is stored at the pair's index (and
     // summed per point afterwards), and every sample writes a basis-parameter partial row of its own.
     int deterministic;
+    // Floats between the feature-gradient copies of neighboring XCDs (0: one array for all of them).
+    int64_t feat_copy_stride;
 };
 
 // First bin whose upper edge is >= v, the last bin when there is none.

@@ -278,6 +278,29 @@ def test_forward_projection_at_the_edges_of_its_tiles(ops, oracle, k, c_in):
     assert np.array_equal(again[~hit], out[~hit])
 
 
+@pytest.mark.parametrize("n,m,per,c_in,k", [(5, 700, 3, 33, 15), (3, 400, 2, 64, 16), (7, 300, 1, 129, 8),
+                                            (40, 900, 4, 70, 15), (2, 130, 1, 50, 33)])
+def test_feature_gradients_of_points_with_many_pairs(ops, oracle, n, m, per, c_in, k):
+    """Few points and many samples (a decoder's way up), on both sides of 64 pairs to a point; odd row widths."""
+    rng = np.random.default_rng(n * m + c_in)
+    pts = rng.uniform(0.0, 0.2, (n, 3)).astype(np.float32)
+    smp = rng.uniform(0.0, 0.2, (m, 3)).astype(np.float32)
+    neigh = np.stack([np.concatenate([rng.permutation(n)[:per] for _ in range(m)]), np.repeat(np.arange(m), per)],
+                     1).astype(np.int32)
+    ends = np.arange(1, m + 1, dtype=np.int32) * per
+    radii = np.full(3, 0.2, np.float32)
+    kp, sigma = synthetic.kernel_points_sphere(1, k)
+    feats = rng.normal(size=(n, c_in)).astype(np.float32)
+    w = rng.normal(0, np.sqrt(1.0 / (k * c_in)), (k * c_in, 20)).astype(np.float32)
+    g = rng.normal(size=(m, 20)).astype(np.float32)
+    exp = oracle.kpconv_grads(pts, feats, smp, neigh, ends, radii, kp, sigma, w, g)
+    # twice: the second call finds the first one's sums in its workspace
+    for _ in range(2):
+        got = ops.kp_conv_grads(t(pts), t(feats), t(smp), t(neigh), t(ends), t(radii), t(kp), sigma, t(w), t(g))
+        for a, e, name in zip(got, exp, ("dW", "dFeat", "dKernelPts", "dPts", "dSamples")):
+            assert relerr(a.cpu().numpy(), e) < GRAD_TOL, name
+
+
 @pytest.mark.parametrize("hidden,mlps,c_in,c_out,distinct", [(16, 1, 64, 128, False), (8, 2, 32, 24, True),
                                                              (16, 1, 3, 16, True), (4, 4, 8, 8, False)])
 def test_mcconv_forward_and_grads(ops, oracle, hidden, mlps, c_in, c_out, distinct):
