@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_tiles.h"
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -32,7 +33,6 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-#define GS_K 32            // reduction elements per step of the split kernel
 #define GS_PLANES 3
 // Operands are scaled by 2^16 (exact) on their way into terms and results back by 2^-32: a third term of the smallest
 // normal number then still is a bf16 number, and even subnormal operands are carried exactly.  What overflows on the
@@ -117,9 +117,7 @@ __device__ __forceinline__ float gemm_dot(const float *__restrict__ a, const flo
 // rows: of two neighboring rows) and splits them in registers.
 //   KC (reduction index contiguous in memory): unit u = (x = u / 4, k / 8 = u % 4), two 16-byte loads;
 //   XC (row / column index contiguous): unit u = (k / 8 = u / (X / W), x = W (u % (X / W))), eight loads of W floats.
-// The wide loads are dword-aligned: any leading dimension.  Rows past the edge read the last row (their results are
-// not stored); an XC pair that straddles the edge reads the next row's first element; the last step of a reduction
-// that is not whole is loaded element by element, with zeros past its end, so nothing outside the operands is touched.
+// The wide loads are dword-aligned: any leading dimension.  Which elements they touch is in gemm_tiles.h.
 //
 // One LDS buffer and two barriers per step, the next step's loads in flight in registers: the two or three workgroups
 // of a CU fill each other's gaps.  Tried and not faster: two steps of loads ahead (no difference); two LDS buffers of
@@ -155,34 +153,27 @@ __device__ __forceinline__ void gs_split(const float (&x)[8], uint4 (&term)[GS_P
     for (int p = 0; p < GS_PLANES; ++p) term[p] = make_uint4(t[p][0], t[p][1], t[p][2], t[p][3]);
 }
 
-template <bool KC, int X> struct SplitOperand {
-    static constexpr int W = (!KC && X >= 96) ? 2 : 1;              // rows per unit load
-    static constexpr int UNITS = X * (GS_K / 8) / W;
-    static constexpr int PASSES = (UNITS + 255) / 256;
+template <bool KC, int X> struct SplitOperand : GemmUnits<KC, X> {
+    typedef GemmUnits<KC, X> Units;
+    static constexpr int W = Units::W, PASSES = Units::PASSES;
     const float *base;                                              // uniform: origin of the current step
     int64_t ld;
     unsigned off[PASSES];                                           // this thread's units, in bytes
     int x_left;                                                     // rows of the operand from the tile's first on
     struct Regs { float v[PASSES][8 * W]; };
 
-    __device__ __forceinline__ static bool active(int i) { return UNITS % 256 == 0 || (int)threadIdx.x + 256 * i < UNITS; }
-    __device__ __forceinline__ static void unit(int i, int &x, int &k8)
-    {
-        const int u = threadIdx.x + 256 * i;
-        if (KC) { x = u / (GS_K / 8); k8 = u % (GS_K / 8); }
-        else { k8 = u / (X / W); x = (u % (X / W)) * W; }
-    }
+    __device__ __forceinline__ static bool active(int i) { return Units::active(threadIdx.x, i); }
+    __device__ __forceinline__ static void unit(int i, int &x, int &k8) { Units::unit(threadIdx.x, i, x, k8); }
     __device__ __forceinline__ void init(const float *origin, int64_t ld_, int64_t x0, int64_t x_end, int64_t k0)
     {
         ld = ld_;
-        base = origin + (KC ? x0 * ld + k0 : k0 * ld + x0);
-        x_left = (int)((x_end - x0) < X ? (x_end - x0) : X);
+        base = origin + Units::origin(x0, k0, ld);
+        x_left = Units::rows_left(x0, x_end);
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) {
             int x, k8;
             unit(i, x, k8);
-            const unsigned xc = (unsigned)(x < x_left ? x : x_left - 1), kk = (unsigned)(k8 * 8);
-            off[i] = (KC ? xc * (unsigned)ld + kk : kk * (unsigned)ld + xc) * 4u;
+            off[i] = Units::offset(x, k8, x_left, (unsigned)ld) * 4u;
         }
     }
     // the step at `base`, which moves on
@@ -210,7 +201,7 @@ template <bool KC, int X> struct SplitOperand {
                 }
             }
         }
-        base += KC ? GS_K : GS_K * ld;
+        base += Units::advance(ld);
     }
     // the last step: k_left elements of the reduction, zeros past them
     __device__ __forceinline__ void load_last(Regs &r, int k_left)
@@ -222,13 +213,10 @@ template <bool KC, int X> struct SplitOperand {
             unit(i, x, k8);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const int k = k8 * 8 + e;
-                const bool in = k < k_left;
-                const int64_t kc = in ? k : k_left - 1;
+                const bool in = k8 * 8 + e < k_left;
 #pragma unroll
                 for (int w = 0; w < W; ++w) {
-                    const int64_t xc = x + w < x_left ? x + w : x_left - 1;
-                    const float q = base[KC ? xc * ld + kc : kc * ld + xc];
+                    const float q = base[Units::checked(x + w, k8 * 8 + e, x_left, k_left, ld)];
                     r.v[i][e * W + w] = in ? q : 0.0f;
                 }
             }
@@ -289,11 +277,9 @@ gemm_f32_split_kernel(GemmArgs g, float *__restrict__ partial)
     ob.init(b, g.ldb, t.bn, g.cols, t.k_begin);
     typename SplitOperand<!AT, BM>::Regs va;
     typename SplitOperand<BT, BN>::Regs vb;
-    const int64_t nk = (t.k_end - t.k_begin + GS_K - 1) / GS_K;
-    // the last step needs no checks when it is whole and no pair of rows straddles an edge
-    const bool whole = (t.k_end - t.k_begin) % GS_K == 0 && (SplitOperand<!AT, BM>::W == 1 || g.rows % 2 == 0) &&
-                       (SplitOperand<BT, BN>::W == 1 || g.cols % 2 == 0);
-    const int nf = (int)(whole ? nk : nk - 1);                      // steps loaded without checks
+    const int64_t nk = gemm_steps(t.k_end - t.k_begin);
+    const int nf = (int)gemm_steps_unchecked(t.k_end - t.k_begin, SplitOperand<!AT, BM>::W, g.rows,
+                                             SplitOperand<BT, BN>::W, g.cols);
     // this wave's LDS traffic is complete, then everyone's (the global loads stay in flight)
     auto lds_barrier = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
     auto multiply = [&]() __attribute__((always_inline)) {

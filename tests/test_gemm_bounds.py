@@ -1,0 +1,47 @@
+"""The fp32 contraction touches nothing outside its operands: the index functions that its kernel calls, walked on the
+CPU over every remainder of a tile, both parities and whole, ragged and split reductions."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def bounds(tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("gemm") / "gemm_bounds.so")
+    subprocess.check_call([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC",
+                           os.path.join(HERE, "gemm_bounds.cpp"), "-o", path])
+    lib = ctypes.CDLL(path)
+    i64 = ctypes.c_int64
+
+    def walk(kc, tile, extent, inner, ld, other_w, other_extent, k_chunk):
+        outside, wrong = i64(), i64()
+        lib.gemm_bounds(int(kc), tile, i64(extent), i64(inner), i64(ld), other_w, i64(other_extent), i64(k_chunk),
+                        ctypes.byref(outside), ctypes.byref(wrong))
+        return outside.value, wrong.value
+    return walk
+
+
+@pytest.mark.parametrize("tile", [128, 96, 64, 32])
+@pytest.mark.parametrize("kc", [False, True])
+def test_every_load_lies_in_its_operand(bounds, kc, tile):
+    for extent in list(range(1, tile + 1)) + list(range(2 * tile + 1, 3 * tile + 1)):
+        for inner, k_chunk in ((32, 32), (64, 64), (33, 64), (95, 96), (96, 32), (100, 64), (1, 32)):
+            for other_w, other_extent in ((1, 5), (2, 6), (2, 5)):
+                for pad in (0, 3):
+                    ld = (inner if kc else extent) + pad
+                    assert bounds(kc, tile, extent, inner, ld, other_w, other_extent, k_chunk) == (0, 0), \
+                        (extent, inner, k_chunk, other_w, other_extent, pad)
+
+
+@pytest.mark.parametrize("kc,tile,extent,inner,ld", [
+    (False, 96, 160, 1024, 160),            # weights of 64 -> 160 channels, 16 basis values
+    (False, 128, 100, 1024, 100), (False, 128, 224, 1024, 224),
+    (False, 128, 720, 4096, 720),           # projection of 48 channels x 15, transposed
+    (False, 128, 1680, 65536, 1680), (True, 128, 65536, 1680, 1680)])
+def test_operands_of_convolutions(bounds, kc, tile, extent, inner, ld):
+    for k_chunk in (inner, 512):
+        assert bounds(kc, tile, extent, inner, ld, 2, 128, k_chunk) == (0, 0)

@@ -86,6 +86,20 @@ def test_gemm_is_as_precise_as_fp32_arithmetic(rows, cols, inner, at, bt):
     assert np.linalg.norm(got - exp) / np.linalg.norm(exp) < np.sqrt(inner / 2 + 1) * 2.0 ** -24
 
 
+# last tiles of an even number of rows or columns, with reductions of whole steps: no load leaves the operands
+# (tests/test_gemm_bounds.py walks the addresses)
+@pytest.mark.parametrize("rows,cols,inner,at,split", [
+    (65536, 224, 1024, 0, 1), (20000, 160, 1024, 0, 1), (57346, 250, 1056, 0, 1), (1680, 256, 16384, 1, 18),
+    (720, 96, 8192, 1, 64), (48, 24, 16384, 1, 200)])
+def test_gemm_at_even_edges_of_wide_tiles(rows, cols, inner, at, split):
+    rng = np.random.default_rng(rows + cols)
+    a = rng.normal(size=(inner, rows) if at else (rows, inner)).astype(np.float32)
+    b = rng.normal(size=(inner, cols)).astype(np.float32)
+    exp = (a.T if at else a).astype(np.float64) @ b.astype(np.float64)
+    # the bound of the test above
+    assert np.linalg.norm(_gemm_f32(a, b, at, 0, split) - exp) / np.linalg.norm(exp) < np.sqrt(inner / 2 + 1) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("rows,cols,inner,split", [(200, 40, 3000, 23), (24, 33, 7327, 57), (600, 130, 1000, 3)])
 def test_gemm_split_reduction_with_many_partial_products(rows, cols, inner, split):
     rng = np.random.default_rng(rows)
