@@ -51,10 +51,11 @@ template <bool KC, int X> struct GemmUnits {
 };
 
 // Steps of a reduction of `count` elements, and how many of them, from the first, are loaded without checks: all where
-// the last one is whole and no unit of two rows (w) straddles an edge.
+// the last one is whole and no unit of two rows (w) straddles an edge.  An empty reduction has no step of either kind.
 GEMM_HD int64_t gemm_steps(int64_t count) { return (count + GS_K - 1) / GS_K; }
 GEMM_HD int64_t gemm_steps_unchecked(int64_t count, int w_a, int64_t rows, int w_b, int64_t cols)
 {
+    if (count == 0) return 0;
     const bool whole = count % GS_K == 0 && (w_a == 1 || rows % 2 == 0) && (w_b == 1 || cols % 2 == 0);
     return whole ? gemm_steps(count) : gemm_steps(count) - 1;
 }

@@ -45,3 +45,9 @@ def test_every_load_lies_in_its_operand(bounds, kc, tile):
 def test_operands_of_convolutions(bounds, kc, tile, extent, inner, ld):
     for k_chunk in (inner, 512):
         assert bounds(kc, tile, extent, inner, ld, 2, 128, k_chunk) == (0, 0)
+
+
+@pytest.mark.parametrize("extent", [128, 129])
+@pytest.mark.parametrize("other_w,other_extent", [(1, 5), (2, 5), (2, 6)])
+def test_an_empty_reduction_has_no_steps(bounds, extent, other_w, other_extent):
+    assert bounds(False, 128, extent, 0, extent, other_w, other_extent, 32) == (0, 0)

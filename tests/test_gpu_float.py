@@ -100,6 +100,17 @@ def test_gemm_at_even_edges_of_wide_tiles(rows, cols, inner, at, split):
     assert np.linalg.norm(_gemm_f32(a, b, at, 0, split) - exp) / np.linalg.norm(exp) < np.sqrt(inner / 2 + 1) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("rows,cols", [(60001, 129), (60000, 128), (30011, 96), (9001, 33), (31, 7)])
+@pytest.mark.parametrize("at,bt", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_of_an_empty_reduction_is_zero(rows, cols, at, bt):
+    from pccnn_lib_amd import _lib
+    operand, out = torch.ones(256, device=DEV), torch.full((rows, cols), float("nan"), device=DEV)
+    _lib.call("pccnn_gemm_f32", _lib.P(operand.data_ptr()), _lib.P(operand.data_ptr()), _lib.P(out.data_ptr()), rows,
+              cols, 0, at, bt, rows if at else 0, 0 if bt else cols, cols, 1, 0, 0, 0, 1, None, 0,
+              _lib.P(torch.cuda.current_stream().cuda_stream))
+    assert not out.any()
+
+
 @pytest.mark.parametrize("rows,cols,inner,split", [(200, 40, 3000, 23), (24, 33, 7327, 57), (600, 130, 1000, 3)])
 def test_gemm_split_reduction_with_many_partial_products(rows, cols, inner, split):
     rng = np.random.default_rng(rows)
