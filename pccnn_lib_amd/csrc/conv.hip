@@ -15,6 +15,7 @@
 // derivative and accumulates point, sample, density and basis-parameter gradients.
 #include "common.h"
 #include "conv_basis.h"
+#include "gemm_tiles.h"
 
 // Sample lists usually come in a spatial order (pooled points and sorted clouds are in cell order), and neighboring
 // samples share most of their neighbors: runs of CONV_XCD_CHUNK consecutive samples go to one XCD (see
@@ -1470,17 +1471,6 @@ extern "C" size_t pccnn_conv_workspace_bytes_deterministic(int64_t n, int64_t m,
            pccnn_align((size_t)t * c_in * sizeof(float)) + by_point_index_bytes(n, t) + 256;
 }
 
-// Split of the sample dimension for d_weights = P^T x dOut with bf16 operands, whose output ([K*Cin, Cout]) has few
-// tiles: bound by its operand traffic, so about four workgroups per CU, with at least 128 samples each.
-static int conv_split_k_bf16(int64_t inner, int64_t co, int num_mlps, int64_t m, size_t workspace_floats)
-{
-    int64_t split = pccnn_ceil_div(1024, pccnn_ceil_div(inner, 64) * pccnn_ceil_div(co, 128) * num_mlps);
-    const int64_t room = (int64_t)(workspace_floats / ((size_t)inner * co * num_mlps));
-    if (split > m / 128) split = m / 128;
-    if (split > room) split = room;
-    return split < 1 ? 1 : (int)split;
-}
-
 // out[m, c_out] = P[m, c_in*k] x W, with the feature axis split over num_mlps independent
 // weight blocks (num_mlps == 1 is the plain product).
 static int contraction_fwd(const float *proj, const float *weights, float *out, int64_t m, int c_in, int k,
@@ -1710,7 +1700,7 @@ static int conv_backward(ConvGeom g, const float *feats, const float *weights, c
             if ((rc = launch_proj_fwd<BASIS>(g, feats, proj_ws, s, bf16)) != PCCNN_OK) return rc;
             proj = proj_ws;
         }
-        const int split = bf16 ? conv_split_k_bf16(inner, co, num_mlps, g.m, splitk_elems)
+        const int split = bf16 ? gemm_bf16_split(inner, co, g.m, num_mlps, splitk_elems)
                                : pccnn_gemm_f32_split(inner, co, g.m, num_mlps, splitk_elems);
         if (bf16)
             rc = pccnn_gemm_bf16((const uint16_t *)proj, g16, d_weights, inner, co, g.m, 1, 0, (int64_t)g.c_in * g.k,

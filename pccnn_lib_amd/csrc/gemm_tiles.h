@@ -1,8 +1,10 @@
-// Which elements of its operands a thread of the fp32 contraction (gemm_f32_split_kernel in gemm.hip) touches, as plain
-// functions: the kernel calls them, and tests/gemm_bounds.cpp walks them on the CPU.
+// Index arithmetic and split rules of the contractions as plain functions: which elements of its operands a thread of the
+// fp32 contraction (gemm_f32_split_kernel in gemm.hip) touches, and into how many parts a reduction is split.  The
+// kernels and their launches call them; tests/gemm_bounds.cpp walks them on the CPU.
 #ifndef PCCNN_GEMM_TILES_H
 #define PCCNN_GEMM_TILES_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #ifdef __HIPCC__
@@ -58,6 +60,24 @@ GEMM_HD int64_t gemm_steps_unchecked(int64_t count, int w_a, int64_t rows, int w
     if (count == 0) return 0;
     const bool whole = count % GS_K == 0 && (w_a == 1 || rows % 2 == 0) && (w_b == 1 || cols % 2 == 0);
     return whole ? gemm_steps(count) : gemm_steps(count) - 1;
+}
+
+// Split of the sample dimension for d_weights = P^T x dOut with bf16 operands (tiles of 64 x 128 or, from 1024 workgroups
+// of those on, 128 x 128): a product bound by its operand traffic, whose output has few tiles.  As many parts as fit on
+// the chip at once, four workgroups per CU, and not one more: 720 x 16 x 65 536 takes 40 us with 1020 workgroups and 55
+// with 1152; parts of 64 samples or more; from 30 000 samples on 64 parts even where they do not fit at once, for the
+// taller tile (2560 x 160 x 120 000: 330 us, 400 with 12 parts; 1920 x 256 x 65 536: 165, 196 with 12), but not
+// before, where the partial sums weigh more than that gains (1920 x 256 x 8192: 58 us with 64 parts, 43 with 17;
+// 2560 x 256 x 20 000: 109 and 78).
+inline int gemm_bf16_split(int64_t rows, int64_t cols, int64_t inner, int batch, size_t workspace_floats)
+{
+    const int64_t tiles = (rows + 63) / 64 * ((cols + 127) / 128) * batch;
+    const int64_t room = (int64_t)(workspace_floats / ((size_t)rows * cols * batch));
+    int64_t split = 1024 / tiles;
+    if (split < 64 && inner >= 30000) split = 64;
+    if (split > inner / 64) split = inner / 64;
+    if (split > room) split = room;
+    return split < 1 ? 1 : (int)split;
 }
 
 #endif

@@ -74,3 +74,8 @@ extern "C" void gemm_bounds(int kc, int tile, int64_t extent, int64_t inner, int
     *outside = tally.outside;
     *wrong = tally.wrong;
 }
+
+extern "C" int bf16_split(int64_t rows, int64_t cols, int64_t inner, int batch, int64_t workspace_floats)
+{
+    return gemm_bf16_split(rows, cols, inner, batch, (size_t)workspace_floats);
+}

@@ -10,16 +10,20 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 @pytest.fixture(scope="module")
-def bounds(tmp_path_factory):
+def library(tmp_path_factory):
     path = str(tmp_path_factory.mktemp("gemm") / "gemm_bounds.so")
     subprocess.check_call([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC",
                            os.path.join(HERE, "gemm_bounds.cpp"), "-o", path])
-    lib = ctypes.CDLL(path)
+    return ctypes.CDLL(path)
+
+
+@pytest.fixture(scope="module")
+def bounds(library):
     i64 = ctypes.c_int64
 
     def walk(kc, tile, extent, inner, ld, other_w, other_extent, k_chunk):
         outside, wrong = i64(), i64()
-        lib.gemm_bounds(int(kc), tile, i64(extent), i64(inner), i64(ld), other_w, i64(other_extent), i64(k_chunk),
+        library.gemm_bounds(int(kc), tile, i64(extent), i64(inner), i64(ld), other_w, i64(other_extent), i64(k_chunk),
                         ctypes.byref(outside), ctypes.byref(wrong))
         return outside.value, wrong.value
     return walk
@@ -51,3 +55,19 @@ def test_operands_of_convolutions(bounds, kc, tile, extent, inner, ld):
 @pytest.mark.parametrize("other_w,other_extent", [(1, 5), (2, 5), (2, 6)])
 def test_an_empty_reduction_has_no_steps(bounds, extent, other_w, other_extent):
     assert bounds(False, 128, extent, 0, extent, other_w, other_extent, 32) == (0, 0)
+
+
+@pytest.mark.parametrize("rows", [9, 48, 64, 65, 720, 1024, 1920, 2560, 10240])
+@pytest.mark.parametrize("cols", [1, 16, 128, 129, 256])
+@pytest.mark.parametrize("batch", [1, 4])
+def test_bf16_weight_gradient_is_split_into_one_round_of_workgroups_or_sixty_four_parts(library, rows, cols, batch):
+    i64 = ctypes.c_int64
+    floats = max(64 * rows * cols * batch, 1 << 20)
+    tiles = -(-rows // 64) * -(-cols // 128) * batch
+    for inner in (1, 63, 64, 1000, 4096, 8192, 20000, 29999, 30000, 65536, 200000):
+        split = library.bf16_split(i64(rows), i64(cols), i64(inner), batch, i64(floats))
+        assert 1 <= split <= max(1, inner // 64) and split * rows * cols * batch <= floats
+        # four workgroups per CU at most ...
+        assert split * tiles <= 1024 or split == 1 or (split == 64 and inner >= 30000)
+        # ... and no fewer parts than 64 where the reduction is long
+        assert inner < 30000 or split >= 64
