@@ -176,36 +176,55 @@ template <bool KC, int X> struct SplitOperand : GemmUnits<KC, X> {
             off[i] = Units::offset(x, k8, x_left, (unsigned)ld) * 4u;
         }
     }
+    // the unit of pass i at `bytes` from the step's origin
+    __device__ __forceinline__ void load_unit(Regs &r, int i, unsigned bytes)
+    {
+        if (KC) {
+            const floatx4u lo = *(const floatx4u *)((const char *)base + bytes);
+            const floatx4u hi = *(const floatx4u *)((const char *)(base + 4) + bytes);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { r.v[i][e] = lo[e]; r.v[i][4 + e] = hi[e]; }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const char *p = (const char *)(base + e * ld) + bytes;
+                if (W == 2) {
+                    const floatx2u q = *(const floatx2u *)p;
+                    r.v[i][2 * e] = q[0];
+                    r.v[i][2 * e + W - 1] = q[1];
+                } else {
+                    r.v[i][e] = *(const float *)p;
+                }
+            }
+        }
+    }
     // the step at `base`, which moves on
     __device__ __forceinline__ void load(Regs &r)
     {
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) {
             if (!active(i)) break;
-            if (KC) {
-                const floatx4u lo = *(const floatx4u *)((const char *)base + off[i]);
-                const floatx4u hi = *(const floatx4u *)((const char *)(base + 4) + off[i]);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { r.v[i][e] = lo[e]; r.v[i][4 + e] = hi[e]; }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const char *p = (const char *)(base + e * ld) + off[i];
-                    if (W == 2) {
-                        const floatx2u q = *(const floatx2u *)p;
-                        r.v[i][2 * e] = q[0];
-                        r.v[i][2 * e + W - 1] = q[1];
-                    } else {
-                        r.v[i][e] = *(const float *)p;
-                    }
-                }
-            }
+            load_unit(r, i, off[i]);
         }
         base += Units::advance(ld);
     }
-    // the last step: k_left elements of the reduction, zeros past them
+    // the last step: k_left elements of the reduction, zeros past them.  Whole units where there are no others (65 536 x
+    // 128 x 48: 14.5 us, 17.0 element by element; 32 768 x 1024 x 16, B transposed: 27 and 33, x 48: 33 and 46)
     __device__ __forceinline__ void load_last(Regs &r, int k_left)
     {
+        if (Units::whole_units(x_left, k_left)) {                   // uniform
+#pragma unroll
+            for (int i = 0; i < PASSES; ++i) {
+                if (!active(i)) break;
+                int x, k8;
+                unit(i, x, k8);
+                const bool in = k8 * 8 < k_left;
+                load_unit(r, i, Units::offset(x, in ? k8 : 0, x_left, (unsigned)ld) * 4u);
+#pragma unroll
+                for (int e = 0; e < 8 * W; ++e) r.v[i][e] = in ? r.v[i][e] : 0.0f;
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) {
             if (!active(i)) break;
@@ -282,9 +301,10 @@ gemm_f32_split_kernel(GemmArgs g, float *__restrict__ partial)
                                              SplitOperand<BT, BN>::W, g.cols);
     // this wave's LDS traffic is complete, then everyone's (the global loads stay in flight)
     auto lds_barrier = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    auto multiply = [&]() __attribute__((always_inline)) {
+    auto multiply = [&](int k_left) __attribute__((always_inline)) {
 #pragma unroll
         for (int ks = 0; ks < GS_K / 16; ++ks) {
+            if (16 * ks >= k_left) break;                           // uniform; zeros
             const int k8 = 2 * ks + h;
             bf16x8 fa[GS_PLANES][TM], fb[GS_PLANES][TN];
 #pragma unroll
@@ -322,9 +342,9 @@ gemm_f32_split_kernel(GemmArgs g, float *__restrict__ partial)
             oa.load(va);
             ob.load(vb);
         }
-        multiply();
+        multiply(GS_K);
     }
-    if (nf < nk) {                                                  // the last step, element by element
+    if (nf < nk) {                                                  // the last step, with checks
         const int k_left = (int)(t.k_end - t.k_begin - (int64_t)nf * GS_K);
         oa.load_last(va, k_left);
         ob.load_last(vb, k_left);
@@ -332,7 +352,7 @@ gemm_f32_split_kernel(GemmArgs g, float *__restrict__ partial)
         SplitOperand<!AT, BM>::park(va, As);
         SplitOperand<BT, BN>::park(vb, Bs);
         lds_barrier();
-        multiply();
+        multiply(k_left);
     }
 
     // With the operands swapped a tile of the accumulator is the transpose of the output tile: lane l holds output

@@ -20,8 +20,8 @@
 //
 // Rows past the tile's or the operand's edge read rows inside it (their results are not stored): a unit of W rows that
 // begins past the edge reads the last W.  A unit of two rows that begins on the last one (odd extents only) reads the
-// next k's first row too, which exists in every step but the last; there, and where a step is not whole, the elements
-// are read one by one, each inside the operand.
+// next k's first row too, which exists in every step but the last.  There, and where a step is not whole, units are read
+// whole only where each is (the empty ones read the step's first), else element by element, each inside the operand.
 template <bool KC, int X> struct GemmUnits {
     static constexpr int W = (!KC && X >= 96) ? 2 : 1;              // rows per unit load
     static constexpr int UNITS = X * (GS_K / 8) / W;
@@ -44,6 +44,8 @@ template <bool KC, int X> struct GemmUnits {
         const unsigned xc = (unsigned)(x < x_left ? x : (x_left >= W ? x_left - W : 0)), kk = (unsigned)(k8 * 8);
         return KC ? xc * ld + kk : kk * ld + xc;
     }
+    // Whether the units of a step of which k_left elements of the reduction are left are all whole or empty.
+    static GEMM_HD bool whole_units(int x_left, int k_left) { return k_left % 8 == 0 && (W == 1 || x_left % 2 == 0); }
     // Element (x, k) of a step of which k_left elements of the reduction are left, or one inside the operand for it.
     static GEMM_HD int64_t checked(int x, int k, int x_left, int k_left, int64_t ld)
     {

@@ -43,10 +43,11 @@ void walk(const Operand &o, int other_w, int64_t other_extent, int64_t k_chunk, 
                         U::unit(thread, i, x, k8);
                         for (int e = 0; e < 8; ++e)
                             for (int w = 0; w < U::W; ++w) {
+                                const int k_left = (int)(k_end - k), in = step < unchecked || k8 * 8 < k_left;
                                 const int64_t element =
-                                    step < unchecked
-                                        ? base + U::offset(x, k8, x_left, (unsigned)o.ld) + (KC ? e : e * o.ld + w)
-                                        : base + U::checked(x + w, k8 * 8 + e, x_left, (int)(k_end - k), o.ld);
+                                    step < unchecked || U::whole_units(x_left, k_left)
+                                        ? base + U::offset(x, in ? k8 : 0, x_left, (unsigned)o.ld) + (KC ? e : e * o.ld + w)
+                                        : base + U::checked(x + w, k8 * 8 + e, x_left, k_left, o.ld);
                                 // (a row that lies in the next tile belongs to that tile)
                                 tally.see(o, element, x + w < x_left ? x0 + x + w : o.extent, k + k8 * 8 + e, k_end);
                             }

@@ -100,6 +100,19 @@ def test_gemm_at_even_edges_of_wide_tiles(rows, cols, inner, at, split):
     assert np.linalg.norm(_gemm_f32(a, b, at, 0, split) - exp) / np.linalg.norm(exp) < np.sqrt(inner / 2 + 1) * 2.0 ** -24
 
 
+# reductions whose last step has eight, sixteen or twenty-four elements, alone and behind whole steps
+@pytest.mark.parametrize("rows,cols,inner", [(57346, 250, 8), (60000, 128, 16), (60001, 129, 24), (30010, 96, 48),
+                                             (58001, 63, 1032), (20000, 32, 1048), (9001, 33, 1064)])
+@pytest.mark.parametrize("at,bt", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_of_reductions_that_end_within_a_step(rows, cols, inner, at, bt):
+    rng = np.random.default_rng(rows + inner)
+    a = rng.normal(size=(inner, rows) if at else (rows, inner)).astype(np.float32)
+    b = rng.normal(size=(cols, inner) if bt else (inner, cols)).astype(np.float32)
+    exp = (a.T if at else a).astype(np.float64) @ (b.T if bt else b).astype(np.float64)
+    # the bound of test_gemm_is_as_precise_as_fp32_arithmetic
+    assert np.linalg.norm(_gemm_f32(a, b, at, bt) - exp) / np.linalg.norm(exp) < np.sqrt(inner / 2 + 1) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("rows,cols", [(60001, 129), (60000, 128), (30011, 96), (9001, 33), (31, 7)])
 @pytest.mark.parametrize("at,bt", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_gemm_of_an_empty_reduction_is_zero(rows, cols, at, bt):
