@@ -132,6 +132,16 @@ def test_gemm_split_reduction_with_many_partial_products(rows, cols, inner, spli
     assert relerr(_gemm_f32(a, b, 1, 0, split), exp) < 1e-5
 
 
+# the sum's threads per element change at 65 536 and 131 072 elements
+@pytest.mark.parametrize("rows,cols", [(512, 128), (513, 128), (720, 91), (1023, 128), (1024, 128)])
+@pytest.mark.parametrize("split", [9, 23])
+def test_gemm_sum_of_partial_products_of_many_elements(rows, cols, split):
+    rng = np.random.default_rng(rows + split)
+    a, b = (rng.normal(size=(1500, n)).astype(np.float32) for n in (rows, cols))
+    exp = a.T.astype(np.float64) @ b.astype(np.float64)
+    assert relerr(_gemm_f32(a, b, 1, 0, split), exp) < 1e-5         # as in the test above
+
+
 def test_gemm_of_huge_tiny_and_non_finite_values():
     # 65 536 rows: the split kernel.  Values that round up to infinity as bf16, infinities and NaNs give what fp32
     # arithmetic gives, in the rows they stand in; rows of very small values keep fp32's relative precision.
