@@ -176,20 +176,21 @@ conv_proj_fwd_kernel(ConvGeom g, const float *__restrict__ feats, void *__restri
     }
 }
 
-// Forward projection of at most 16 basis values on the matrix cores: P[k][f] = sum over the pairs of w[k][t] F[t][f] is
+// Forward projection of 9 to 16 basis values on the matrix cores: P[k][f] = sum over the pairs of w[k][t] F[t][f] is
 // a product per sample with the pairs as its inner dimension, four of them per v_mfma_f32_16x16x4_f32.  One wavefront
 // per (sample, 64 features), lane = (q = lane / 16, c = lane % 16): it evaluates basis value c of pair 4 i + q and
 // loads feature 16 u + c of that pair's row, which are the operands as the instruction takes them; no value passes
 // through LDS but the pairs' geometry.  Products and sums are fp32 as on the vector ALU.
-// conv_proj_fwd_kernel, which takes 17 and more basis values, is bound by its broadcast reads of the basis values from
-// LDS and by the vector ALU; at 16 and fewer it was the slower one at every size measured, us there / here: 65 536
-// samples, 14.4 pairs, 64 features x 16: 89 / 81, bf16 out 84 / 72; 65 536, 18.1, 128 x 15: 235 / 186; 37 675, 21.5,
-// 48 x 15: 73 / 55; 120 000, 13.5, 128 x 15: 355 / 319 (the write of 922 MB).  What bounds it now is that write.
-template <int BASIS, int KPAD, bool BF16>
+// conv_proj_fwd_kernel, which takes the others, is bound by its broadcast reads of the basis values from LDS and by the
+// vector ALU, us there / here: 65 536 samples, 14.4 pairs, 64 features x 16: 89 / 81, bf16 out 84 / 72; 65 536, 18.1,
+// 128 x 15: 235 / 186; 37 675, 21.5, 48 x 15: 73 / 55; 120 000, 13.5, 128 x 15: 355 / 319 (the write of 922 MB).  What
+// bounds it now is that write.  With 8 basis values half of every tile and of the lanes' basis evaluations would be
+// padding: 65 536 samples, 64 features x 8: 64 / 72, bf16 out 60 / 69; 128 x 8: 122 / 137; 10 500, 128 x 8: 31 / 34.
+template <int BASIS, bool BF16>
 __global__ void __launch_bounds__(64)
 conv_proj_fwd_mfma_kernel(ConvGeom g, const float *__restrict__ feats, void *__restrict__ proj_out)
 {
-    static_assert(KPAD == 8 || KPAD == 16, "one 16-row tile of basis values");
+    constexpr int KPAD = 16;                            // one 16-row tile of basis values
     constexpr bool GEOM = BASIS != BASIS_EXPLICIT;      // explicit basis values need no positions
     constexpr int STEPS = 2;                            // groups of four pairs in flight
     __shared__ float4 geo_lds[GEOM ? 64 : 1];           // (offset, density) of the chunk's pairs
@@ -268,7 +269,6 @@ conv_proj_fwd_mfma_kernel(ConvGeom g, const float *__restrict__ feats, void *__r
     const int64_t dst_at = ((int64_t)s * g.c_in + f0) * g.k;
     if (g.k == KPAD) {
         // four neighboring basis values per lane: every store instruction writes one contiguous run
-        if (4 * q >= KPAD) return;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int f = 16 * u + c;
@@ -1343,19 +1343,16 @@ static int launch_proj_fwd(const ConvGeom &g, const float *feats, void *proj, hi
         if (bf16) conv_proj_fwd_kernel<BASIS, KP, true><<<grid, 64, 0, s>>>(g, feats, proj);  \
         else conv_proj_fwd_kernel<BASIS, KP, false><<<grid, 64, 0, s>>>(g, feats, proj);      \
     } while (0)
-#define MFMA_GO(KP)                                                                              \
-    do {                                                                                         \
-        if (bf16) conv_proj_fwd_mfma_kernel<BASIS, KP, true><<<grid, 64, 0, s>>>(g, feats, proj);  \
-        else conv_proj_fwd_mfma_kernel<BASIS, KP, false><<<grid, 64, 0, s>>>(g, feats, proj);      \
-    } while (0)
     switch (kpad_of(g.k)) {
-    case 8: MFMA_GO(8); break;
-    case 16: MFMA_GO(16); break;
+    case 8: PROJ_GO(8); break;
+    case 16:
+        if (bf16) conv_proj_fwd_mfma_kernel<BASIS, true><<<grid, 64, 0, s>>>(g, feats, proj);
+        else conv_proj_fwd_mfma_kernel<BASIS, false><<<grid, 64, 0, s>>>(g, feats, proj);
+        break;
     case 32: PROJ_GO(32); break;
     default: PROJ_GO(64); break;
     }
 #undef PROJ_GO
-#undef MFMA_GO
     PCCNN_LAUNCH_CHECK();
     return PCCNN_OK;
 }
