@@ -1615,10 +1615,13 @@ static int conv_backward(ConvGeom g, const float *feats, const float *weights, c
     // array.  One copy of it per XCD, added up afterwards, in the buffer of the projection, which is free by then:
     // 4800 points, 1.62 M pairs (337 to a point), 128 features: 815 -> 710 us, the sum 5 us.  With 14 pairs to a point
     // and 16.8 MB of gradients the kernel gains nothing (255 us either way) and clearing and adding the copies costs
-    // 40 us; from 64 pairs to a point on, that cost is below a tenth of the atomics' own.
+    // 40 us; whole training steps of 120 000 samples, 128 features: 2040 -> 2014 us at 92 pairs to a point, 2155 -> 2102
+    // at 184, 2264 -> 2144 at 265; 40 features: 816 -> 798 at 92.  Below some 8 M atomics (pairs x features) the two
+    // launches cost what they save: 2000 samples, 128 features 123 -> 129, 8000 samples, 40 features 125 -> 129 at 131
+    // pairs to a point, 8000 samples, 128 features 236 -> 219.
     const int64_t copy_stride = (g.n * g.c_in + 3) / 4 * 4;
     const bool copies = !rows_route && want_f && g.c_in > 32 && g.m > 0 && g.t / 64 >= g.n &&
-                        copy_stride <= g.m * g.c_in * g.k / PCCNN_XCDS;
+                        g.t * g.c_in >= (1 << 23) && copy_stride <= g.m * g.c_in * g.k / PCCNN_XCDS;
     g.feat_copy_stride = copies ? copy_stride : 0;
     PccnnArena arena(workspace, workspace_bytes);
     const int64_t partial_rows = det ? g.m : PARAM_ROWS;

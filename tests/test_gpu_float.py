@@ -349,6 +349,28 @@ def test_feature_gradients_of_points_with_many_pairs(ops, oracle, n, m, per, c_i
             assert relerr(a.cpu().numpy(), e) < GRAD_TOL, name
 
 
+# on both sides of 2^23 pair features, odd row widths, with and without a gradient of the weights
+@pytest.mark.parametrize("n,m,c_in,k", [(333, 42366, 33, 5), (701, 42367, 33, 16), (90, 12000, 129, 9), (1000, 11000, 128, 8)])
+def test_feature_gradients_of_few_points_and_millions_of_pair_features(ops, oracle, n, m, c_in, k):
+    rng = np.random.default_rng(n + m)
+    per = 6
+    pts = rng.uniform(0.0, 0.2, (n, 3)).astype(np.float32)
+    smp = rng.uniform(0.0, 0.2, (m, 3)).astype(np.float32)
+    neigh = np.stack([(rng.integers(0, n, m)[:, None] + np.arange(per) * 7).ravel() % n, np.repeat(np.arange(m), per)],
+                     1).astype(np.int32)
+    ends = np.arange(1, m + 1, dtype=np.int32) * per
+    radii = np.full(3, 0.2, np.float32)
+    kp, sigma = synthetic.kernel_points_sphere(1, k)
+    feats = rng.normal(size=(n, c_in)).astype(np.float32)
+    w = rng.normal(0, np.sqrt(1.0 / (k * c_in)), (k * c_in, 8)).astype(np.float32)
+    g = rng.normal(size=(m, 8)).astype(np.float32)
+    args = (t(pts), t(feats), t(smp), t(neigh), t(ends), t(radii), t(kp), sigma, t(w), t(g))
+    exp = oracle.kpconv_grads(pts, feats, smp, neigh, ends, radii, kp, sigma, w, g)[1]
+    for mask in (ops.GRAD_ALL, ops.GRAD_FEATS):
+        got = ops.kp_conv_grads(*args, grad_mask=mask)[1]
+        assert relerr(got.cpu().numpy(), exp) < GRAD_TOL
+
+
 @pytest.mark.parametrize("hidden,mlps,c_in,c_out,distinct", [(16, 1, 64, 128, False), (8, 2, 32, 24, True),
                                                              (16, 1, 3, 16, True), (4, 4, 8, 8, False)])
 def test_mcconv_forward_and_grads(ops, oracle, hidden, mlps, c_in, c_out, distinct):
