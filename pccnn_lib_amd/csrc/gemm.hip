@@ -99,12 +99,37 @@ __device__ __forceinline__ float *gemm_output(const GemmArgs &g, const GemmTile 
     return g.c + (int64_t)t.batch * g.stride_c;
 }
 
-// One element of the product by fp32 multiply-adds, in order.
-__device__ __forceinline__ float gemm_dot(const float *__restrict__ a, const float *__restrict__ b, int64_t a_step,
-                                          int64_t b_step, int64_t count)
+// A 32 x 32 tile of the product by one wavefront on the fp32 matrix instructions, operands straight from memory (`a` and
+// `b`: this lane's row and column; `h`: its half, which takes k = 4 h + e of every eight).  Ends early once every sum
+// that is wanted (bit v: register v of this lane) is NaN.  Few registers rather than many loads in flight: it must not
+// cost the kernel around it a wavefront.
+template <bool AT, bool BT>
+__device__ __forceinline__ floatx16 gemm_tile_f32(const float *__restrict__ a, const float *__restrict__ b, int64_t lda,
+                                                  int64_t ldb, int h, int64_t k_begin, int64_t k_end, unsigned wanted)
 {
-    float s = 0.0f;
-    for (int64_t k = 0; k < count && s == s; ++k) s = fmaf(a[k * a_step], b[k * b_step], s);
+    constexpr int AHEAD = 2;
+    floatx16 s;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] = 0.0f;
+#pragma unroll 1
+    for (int64_t k0 = k_begin; k0 < k_end; k0 += 8 * AHEAD) {
+        float fa[4 * AHEAD], fb[4 * AHEAD];
+#pragma unroll
+        for (int e = 0; e < 4 * AHEAD; ++e) {
+            const int64_t k = k0 + 8 * (e / 4) + 4 * h + e % 4;
+            const bool in = k < k_end;
+            const int64_t kc = in ? k : k_end - 1;
+            fa[e] = a[AT ? kc * lda : kc];
+            fb[e] = b[BT ? kc : kc * ldb];
+            if (!in) fa[e] = fb[e] = 0.0f;
+        }
+#pragma unroll
+        for (int e = 0; e < 4 * AHEAD; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], s, 0, 0, 0);
+        bool done = true;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) done = done && (s[v] != s[v] || !(wanted >> v & 1));
+        if (__all(done)) break;
+    }
     return s;
 }
 
@@ -363,11 +388,12 @@ gemm_f32_split_kernel(GemmArgs g, float *__restrict__ partial)
     lds_barrier();                                                  // the fragments of the last step have been read
     float *stage = (float *)lds + wave * (32 * GS_STAGE_LD);
     const int srow = lane >> 3, scol = (lane & 7) * 4;
-    bool finite = true;
+    unsigned bad = 0;                                               // uniform: tiles with a result that is not finite
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
+            bool finite = true;
 #pragma unroll
             for (int gq = 0; gq < 4; ++gq) {
                 floatx4 v;
@@ -380,6 +406,7 @@ gemm_f32_split_kernel(GemmArgs g, float *__restrict__ partial)
                 }
                 *(floatx4 *)(stage + r * GS_STAGE_LD + 8 * gq + 4 * h) = v;
             }
+            if (__any(!finite)) bad |= 1u << (i * TN + j);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             const int64_t col = t.bn + (wn * TN + j) * 32 + scol;
 #pragma unroll
@@ -397,17 +424,32 @@ gemm_f32_split_kernel(GemmArgs g, float *__restrict__ partial)
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
     // An infinite operand (or one that rounds up to infinity as bf16) makes its terms' products infinity times zero.
-    // Results that are not finite are computed again by plain multiply-adds, which give what fp32 arithmetic gives.
-    if (__any(!finite)) {
+    // Results that are not finite are computed again, a tile at a time, by the fp32 matrix instructions, which give what
+    // fp32 arithmetic gives.  65 536 x 128 x 1024 (116 us): with one infinite weight 340 us, with an infinite column of
+    // them 130 (its results are NaN at once), with infinities everywhere 660; one lane for one element took 640, 130
+    // and 18 000.
+    if (bad != 0) {
         __threadfence_block();
-        for (int e = 0; e < TM * TN * 16; ++e) {
-            const int tile = e / 16, v = e % 16;
-            const int64_t row = t.bm + (wm * TM + tile / TN) * 32 + r;
-            const int64_t col = t.bn + (wn * TN + tile % TN) * 32 + 8 * (v / 4) + 4 * h + v % 4;
-            if (row >= g.rows || col >= g.cols || fabsf(cbase[row * ldc + col]) <= 3.402823466e38f) continue;
-            cbase[row * ldc + col] = gemm_dot(a + (AT ? t.k_begin * g.lda + row : row * g.lda + t.k_begin),
-                                              b + (BT ? col * g.ldb + t.k_begin : t.k_begin * g.ldb + col),
-                                              AT ? g.lda : 1, BT ? 1 : g.ldb, t.k_end - t.k_begin);
+#pragma unroll 1
+        for (int tile = 0; tile < TM * TN; ++tile) {
+            if (!(bad >> tile & 1)) continue;
+            const int64_t row0 = t.bm + (wm * TM + tile / TN) * 32, col0 = t.bn + (wn * TN + tile % TN) * 32;
+            const int64_t row = row0 + r < g.rows ? row0 + r : g.rows - 1, col = col0 + r < g.cols ? col0 + r : g.cols - 1;
+            // register v of lane l: row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32 of the tile
+            unsigned wanted = 0;
+#pragma unroll 2
+            for (int v = 0; v < 16; ++v) {
+                const int64_t orow = row0 + 8 * (v / 4) + 4 * h + v % 4;
+                if (orow < g.rows && col0 + r < g.cols && !(fabsf(cbase[orow * ldc + col0 + r]) <= 3.402823466e38f))
+                    wanted |= 1u << v;
+            }
+            const floatx16 s = gemm_tile_f32<AT, BT>(a + (AT ? row : row * g.lda), b + (BT ? col * g.ldb : col), g.lda,
+                                                     g.ldb, h, t.k_begin, t.k_end, wanted);
+            int64_t ld = ldc;
+            asm volatile("" : "+s"(ld));                            // the addresses anew, not kept over the loop
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                if (wanted >> v & 1) cbase[(row0 + 8 * (v / 4) + 4 * h + v % 4) * ld + col0 + r] = s[v];
         }
     }
 }

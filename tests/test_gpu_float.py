@@ -173,6 +173,30 @@ def test_gemm_of_huge_tiny_and_non_finite_values():
     assert relerr(got[rest], exp[rest]) < 1e-5
 
 
+# every tile of the split kernel, in every layout, at ragged edges; and the short kernel
+@pytest.mark.parametrize("rows,cols,inner", [(60001, 130, 70), (33333, 95, 64), (57346, 64, 33), (30001, 31, 1030),
+                                             (9001, 129, 40), (70, 35, 90)])
+@pytest.mark.parametrize("at,bt", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_of_non_finite_values_in_every_layout(rows, cols, inner, at, bt):
+    rng = np.random.default_rng(rows)
+    a = rng.uniform(0.5, 1.0, (rows, inner)).astype(np.float32)
+    b = rng.uniform(0.5, 1.0, (inner, cols)).astype(np.float32)
+    a[17, inner - 1] = np.inf
+    a[rows - 1, 3] = -np.inf
+    b[5, cols - 1] = np.inf
+    b[2, 7] = np.nan
+    a[40], b[:, 20] = 1e20, 1e20                # their product overflows, each with the others stays in range
+    a[50, 0], b[0, 21] = 2.0 ** 125, 2.0 ** -120
+    with np.errstate(all="ignore"):
+        exp = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    got = _gemm_f32(np.ascontiguousarray(a.T) if at else a, np.ascontiguousarray(b.T) if bt else b, at, bt)
+    assert np.array_equal(np.isnan(got), np.isnan(exp))
+    assert np.array_equal(np.isposinf(got), np.isposinf(exp)) and np.array_equal(np.isneginf(got), np.isneginf(exp))
+    fine = np.isfinite(exp)
+    # positive products: relative error of every element at most inner + 1 roundings
+    assert np.all(np.abs(got[fine] - exp[fine]) <= (inner + 1) * 2.0 ** -24 * np.abs(exp[fine]))
+
+
 @pytest.mark.parametrize("m,mlps,inner,co", [(200, 2, 48, 24), (256, 2, 208, 128), (32768, 3, 192, 128)])
 def test_gemm_batched_strided(m, mlps, inner, co):
     # the second and third shapes have full tiles: the kernel without bounds checks, 64-row and 128-row tiles
