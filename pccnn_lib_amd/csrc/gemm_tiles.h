@@ -54,6 +54,9 @@ template <bool KC, int X> struct GemmUnits {
     }
 };
 
+// Whether the byte offsets of a tile of `rows` rows (or columns) fit into 32 bits.
+inline bool gemm_tile_fits(int rows, int64_t ld) { return ld < (((int64_t)1 << 32) - 256) / 4 / (rows < GS_K ? GS_K : rows); }
+
 // Steps of a reduction of `count` elements, and how many of them, from the first, are loaded without checks: all where
 // the last one is whole and no unit of two rows (w) straddles an edge.  An empty reduction has no step of either kind.
 GEMM_HD int64_t gemm_steps(int64_t count) { return (count + GS_K - 1) / GS_K; }

@@ -41,6 +41,9 @@ void walk(const Operand &o, int other_w, int64_t other_extent, int64_t k_chunk, 
                     for (int i = 0; i < U::PASSES && U::active(thread, i); ++i) {
                         int x, k8;
                         U::unit(thread, i, x, k8);
+                        // the kernel's offsets are 32-bit bytes
+                        const uint64_t bytes = 4 * ((uint64_t)(KC ? X - 1 : 24) * (uint64_t)o.ld + GS_K + X);
+                        if (gemm_tile_fits(X, o.ld) && bytes >> 32) ++tally.outside;
                         for (int e = 0; e < 8; ++e)
                             for (int w = 0; w < U::W; ++w) {
                                 const int k_left = (int)(k_end - k), in = step < unchecked || k8 * 8 < k_left;
@@ -80,3 +83,5 @@ extern "C" int bf16_split(int64_t rows, int64_t cols, int64_t inner, int batch, 
 {
     return gemm_bf16_split(rows, cols, inner, batch, (size_t)workspace_floats);
 }
+
+extern "C" int tile_fits(int rows, int64_t ld) { return gemm_tile_fits(rows, ld); }

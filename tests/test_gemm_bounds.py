@@ -51,6 +51,15 @@ def test_operands_of_convolutions(bounds, kc, tile, extent, inner, ld):
         assert bounds(kc, tile, extent, inner, ld, 2, 128, k_chunk) == (0, 0)
 
 
+@pytest.mark.parametrize("tile", [128, 96, 64, 32])
+@pytest.mark.parametrize("kc", [False, True])
+def test_the_longest_rows_a_tile_takes(bounds, library, kc, tile):
+    fits = lambda ld: library.tile_fits(tile, ctypes.c_int64(ld))
+    ld = max(x for x in range((1 << 30) // tile - 64, (1 << 30) // tile + 1) if fits(x))
+    assert ld >= 1 << 22 and not fits(ld + 1) and not fits(1 << 40)
+    assert bounds(kc, tile, 2 * tile + 2, 100, ld, 1, 5, 64) == (0, 0)
+
+
 @pytest.mark.parametrize("extent", [128, 129])
 @pytest.mark.parametrize("other_w,other_extent", [(1, 5), (2, 5), (2, 6)])
 def test_an_empty_reduction_has_no_steps(bounds, extent, other_w, other_extent):

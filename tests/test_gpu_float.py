@@ -173,6 +173,23 @@ def test_gemm_of_huge_tiny_and_non_finite_values():
     assert relerr(got[rest], exp[rest]) < 1e-5
 
 
+# the widest tiles' offsets fit into 32 bits up to rows of about 2^23, those of 64 x 64 tiles up to 2^24
+@pytest.mark.parametrize("ld", [(1 << 23) - 64, (1 << 23) + 64, (1 << 24) + 64])
+@pytest.mark.parametrize("at", [0, 1])
+def test_gemm_of_operands_with_long_rows(ld, at):
+    from pccnn_lib_amd import _lib
+    rng = np.random.default_rng(ld % 1000 + at)
+    rows, cols, inner = 130, 16500, 70
+    a = rng.normal(size=(inner, rows) if at else (rows, inner)).astype(np.float32)
+    b = rng.normal(size=(inner, cols)).astype(np.float32)
+    wide = torch.empty(a.shape[0] * ld, dtype=torch.float32, device=DEV)
+    wide.as_strided(a.shape, (ld, 1)).copy_(t(a))
+    tb, tc = t(b), torch.full((rows, cols), float("nan"), device=DEV)
+    _lib.call("pccnn_gemm_f32", _lib.P(wide.data_ptr()), _lib.P(tb.data_ptr()), _lib.P(tc.data_ptr()), rows, cols, inner,
+              at, 0, ld, cols, cols, 1, 0, 0, 0, 1, None, 0, _lib.P(torch.cuda.current_stream().cuda_stream))
+    assert relerr(tc.cpu().numpy(), (a.T if at else a).astype(np.float64) @ b.astype(np.float64)) < 1e-5
+
+
 # every tile of the split kernel, in every layout, at ragged edges; and the short kernel
 @pytest.mark.parametrize("rows,cols,inner", [(60001, 130, 70), (33333, 95, 64), (57346, 64, 33), (30001, 31, 1030),
                                              (9001, 129, 40), (70, 35, 90)])
