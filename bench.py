@@ -170,7 +170,7 @@ def config3_leg(lib, dev, timed, steps, warmup, with_cpu):
            "kernels_us": {kk: round(1e3 * v[1] / v[0], 2) for kk, v in kernels.items()},
            "roofline": {"kernel": "gemm_f32_split_kernel (all three products)", "bound": "mfma", "achieved": tflops,
                         "peak": MFMA_SPLIT_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": tflops / MFMA_SPLIT_PEAK_TFLOPS,
-                        "traffic": traffic("config3", "contraction_f32"), "flops_per_launch": flops,
+                        "traffic": traffic("config3", "gemm_f32_split_kernel"), "flops_per_launch": flops,
                         "avg_launch_ms": g_avg, "launches": g_n,
                         "shapes": "P[65536,1920] W[1920,256]; P^T dOut; dOut W^T (mean of the three launches)"}}
     # the two projection kernels of this step against HBM (bytes as for config 2: pairs, offsets, coordinates and
@@ -178,7 +178,7 @@ def config3_leg(lib, dev, timed, steps, warmup, with_cpu):
     # per-pair point gradients out)
     geo = 8.0 * pairs + 4.0 * m + 12.0 * 2 * m + 4.0 * m * c_in
     proj = 4.0 * m * c_in * k
-    for key, name, alg in (("proj_fwd", "conv_proj_fwd_kernel", geo + proj),
+    for key, name, alg in (("proj_fwd", "conv_proj_fwd_mfma_kernel", geo + proj),
                            ("proj_bwd", "conv_proj_bwd_kernel", geo + proj + 4.0 * m * c_in + 4.0 * pairs * k + 16.0 * pairs)):
         k_n, k_ms = kernels.get(key, (0, 0.0))
         avg = k_ms / max(k_n, 1)
@@ -540,7 +540,7 @@ def main():
     gemm_tflops = gemm_flops / (gemm_avg_ms * 1e-3) / 1e12 if gemm_n else 0.0
     roofline = {"kernel": "gemm_f32_split_kernel (all three products)", "bound": "mfma", "achieved": gemm_tflops,
                 "peak": MFMA_SPLIT_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": gemm_tflops / MFMA_SPLIT_PEAK_TFLOPS,
-                "traffic": traffic("config2", "contraction_f32"), "flops_per_launch": gemm_flops, "avg_launch_ms": gemm_avg_ms,
+                "traffic": traffic("config2", "gemm_f32_split_kernel"), "flops_per_launch": gemm_flops, "avg_launch_ms": gemm_avg_ms,
                 "launches": gemm_n}
 
     # ---- the two projection kernels against HBM bandwidth.  Algorithmic bytes, forward: pairs 8T + offsets 4M +
@@ -552,7 +552,7 @@ def main():
     proj_bytes = 4.0 * m * kdim
     rooflines_proj = {}
     for key, name, alg, moved in (
-            ("proj_fwd", "conv_proj_fwd_kernel", geo_bytes + proj_bytes, traffic("config2", "conv_proj_fwd_kernel")),
+            ("proj_fwd", "conv_proj_fwd_mfma_kernel", geo_bytes + proj_bytes, traffic("config2", "conv_proj_fwd_mfma_kernel")),
             ("proj_bwd", "conv_proj_bwd_kernel", geo_bytes + proj_bytes + 4.0 * m * wl["c_in"] +
              4.0 * t_pairs * wl["hidden"] + 16.0 * t_pairs, traffic("config2", "conv_proj_bwd_kernel"))):
         k_n, k_ms = conv_kernels.get(key, (0, 0.0))
