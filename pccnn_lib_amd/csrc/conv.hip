@@ -2,12 +2,15 @@
 // the host entry points that chain them with the fp32 contraction.
 //
 // Forward, per sample s:  P[s][f][k] = sum over the pairs t of s of  F[n_t][f] * w[t][k]
-//   * one wavefront per (sample, block of 64 input features): lane l owns feature f = 64*fb + l
-//     and keeps the K partial sums of its feature in registers;
-//   * the pair geometry (neighbor id, normalised offset, density) of up to 64 pairs is loaded
-//     lane-parallel; the basis values w[t][0..K) of the chunk are evaluated once, K lanes per pair,
+//   * one wavefront per (sample, block of 64 input features); the pair geometry (neighbor id,
+//     normalised offset, density) of up to 64 pairs is loaded lane-parallel;
+//   * 9 to 16 basis values: a matrix product per sample with the pairs as its inner dimension
+//     (conv_proj_fwd_mfma_kernel);
+//   * others: lane l owns feature f = 64*fb + l and keeps the K partial sums of its feature in
+//     registers; the basis values w[t][0..K) of the chunk are evaluated once, K lanes per pair,
 //     and staged in LDS, from where every lane reads them as broadcasts, while the feature row of
-//     each neighbor is one coalesced read;
+//     each neighbor is one coalesced read (conv_proj_fwd_kernel);
+//   * at most 32 features: several pairs side by side (conv_proj_fwd_narrow_kernel);
 //   * P is stored k-fastest, i.e. row f*K + k of the contraction, then out = P x W on MFMA.
 // Backward: dP = dOut x W^T and dW = P^T x dOut on MFMA; a second per-sample walk turns dP into
 // feature gradients (coalesced float atomics per neighbor row) and per-pair basis gradients
@@ -159,10 +162,10 @@ conv_proj_fwd_kernel(ConvGeom g, const float *__restrict__ feats, void *__restri
     } else {
         float *dst = (float *)proj_out + dst_at;
         if (g.k == KPAD) {
-            // whole lines that nothing reads before the next kernel: stored past the L2 (65 536 samples x 64 features
-            // x 16: 85 -> 80 us, the contraction behind it 2 us slower).
-            // Not for the bf16 tile: half the size, much of it is still in cache when the contraction reads it
-            // (40 -> 49 us with such stores).
+            // whole lines that nothing reads before the next kernel: stored past the L2 (65 536 samples x 128 features
+            // x 8: 138 -> 122 us, with the contraction 213 -> 186; 64 features x 32: 191 -> 203, with the
+            // contraction 370 -> 355).  Not for the bf16 tile: half the size, much of it is still in cache when the
+            // contraction reads it.
             for (int i = lane; i < nf * (KPAD / 4); i += 64) {
                 const floatx4_t v = ((const floatx4_t *)tile)[i];
                 __builtin_nontemporal_store(v, &((floatx4_t *)dst)[i]);

@@ -14,12 +14,13 @@
 // float64, relative to the result's norm, this kernel / the fp32 matrix instructions: reduction of 128: 1.6e-7 /
 // 2.0e-7, 1024: 4.9e-7 / 5.7e-7, 1920: 2.6e-7 / 7.8e-7, 3855 of 65 536: 3.9e-7 / 1.1e-6.
 //
-// Measured, before (128 x 128 and 64 x 128 tiles of fp32 matrix instructions) and now, us: 65 536 x 128 x 1024 138 ->
-// 109, its transposes 165 -> 121 and 149 -> 119; 65 536 x 256 x 1920 483 -> 368 (175 TFLOP/s; the fp32 instructions'
-// peak is 157), transposes 522 -> 370 and 515 -> 391; 120 000 x 64 x 1920 541 -> 247; 37 675 x 96 x 720 84 -> 55;
-// 40 000 x 205 x 645 (odd leading dimension) 207 -> 91; 24 x 33 x 7327 138 -> 10; 346 x 256 x 1024 51 -> 11.
-// The large ones are bound by the matrix pipe at the clock that its power allows (counters: 54 % of the cycles at
-// 1.96 GHz; the library's bf16 product reaches 1.34 PFLOP/s on this part, this kernel 1.05 of the six products).
+// Measured, before (128 x 128 and 64 x 128 tiles of fp32 matrix instructions) and now, launches in a row, us: 65 536 x
+// 128 x 1024 174 -> 118, its transposes 171 -> 126 and 162 -> 130; 65 536 x 256 x 1920 493 -> 384 (168 TFLOP/s; the
+// fp32 instructions' peak is 157), transposes 533 -> 369 and 512 -> 397; 120 000 x 64 x 1920 536 -> 249; 37 675 x 96 x
+// 720 89 -> 60; 40 000 x 205 x 645 (odd leading dimension) 169 -> 97; 24 x 33 x 7327 136 -> 9; 346 x 256 x 1024 51 -> 11.
+// The large ones fill no pipe: counters give 47 to 60 % of the SIMD cycles to the matrix pipe and 31 to 42 % to vector
+// instructions, at a clock of about 1.8 GHz; a wavefront splits, hands over and multiplies in turn, and the two or
+// three of a SIMD overlap in part.  The six products run at 1.0 PFLOP/s.
 #include <type_traits>
 
 #include "common.h"
@@ -145,10 +146,10 @@ __device__ __forceinline__ floatx16 gemm_tile_f32(const float *__restrict__ a, c
 // The wide loads are dword-aligned: any leading dimension.  Which elements they touch is in gemm_tiles.h.
 //
 // One LDS buffer and two barriers per step, the next step's loads in flight in registers: the two or three workgroups
-// of a CU fill each other's gaps.  Tried and not faster: two steps of loads ahead (no difference); two LDS buffers of
+// of a CU fill each other's gaps.  Tried and not taken: two steps of loads ahead (no difference); two LDS buffers of
 // 16 with one barrier and the split between the MFMAs of the same wavefront (361 against 364 us at 65 536 x 256 x
-// 1920, slower on narrow tiles and spilling with both operands XC); 256 x 128 tiles (324 there, 118 against 107 at
-// 65 536 x 128 x 1024, 483 against 368 with both operands XC).
+// 1920, slower on narrow tiles and spilling with both operands XC); 256 x 128 tiles everywhere (faster there, 324
+// against 364, slower at 65 536 x 128 x 1024, 118 against 107, and with both operands XC, 483 against 368).
 __device__ __forceinline__ int gs_slot(int x, int k8) { return x ^ ((x >> 3) & 1) ^ (k8 << 1); }
 
 __device__ __forceinline__ uint32_t gs_pack(float lo, float hi)
@@ -456,7 +457,8 @@ gemm_f32_split_kernel(GemmArgs g, float *__restrict__ partial)
 
 // ---------------------------------------------------------------------------------------------------------------
 // Short kernel: products too small to fill the chip with the tiles above (up to 128 of them; 2048 x 32 x 480: 27 -> 7
-// us, where 16 workgroups of the wide tile take 17).  A workgroup of 8 wavefronts owns 32 rows
+// us, where 16 workgroups of the wide tile take 17; long reductions with 32 to 128 tiles, before and now: 1000 x 256 x
+// 2560 120 -> 23, 2048 x 256 x 1920 70 -> 37, 4096 x 128 x 2560 92 -> 46).  A workgroup of 8 wavefronts owns 32 rows
 // and 32 TN columns and splits the reduction: wavefront w takes the groups of eight k number w, w + 8, ...  Operands
 // go straight from memory to the fp32 MFMAs (v_mfma_f32_32x32x2_f32: lane half h takes k = 4 h + e of a group in the
 // e-th of its four MFMAs), four groups requested together; the partial tiles meet in LDS, added in order.

@@ -33,7 +33,8 @@ def bounds(library):
 @pytest.mark.parametrize("kc", [False, True])
 def test_every_load_lies_in_its_operand(bounds, kc, tile):
     for extent in list(range(1, tile + 1)) + list(range(2 * tile + 1, 3 * tile + 1)):
-        for inner, k_chunk in ((32, 32), (64, 64), (33, 64), (95, 96), (96, 32), (100, 64), (1, 32), (8, 32), (16, 32), (24, 32), (56, 64)):
+        for inner, k_chunk in ((32, 32), (64, 64), (33, 64), (95, 96), (96, 32), (100, 64), (1, 32),
+                               (8, 32), (16, 32), (24, 32), (56, 64)):
             for other_w, other_extent in ((1, 5), (2, 6), (2, 5)):
                 for pad in (0, 3):
                     ld = (inner if kc else extent) + pad

@@ -29,13 +29,14 @@ def _cloud(models, batch, num_pts):
 @pytest.mark.parametrize("rows,cols,inner,at,bt,split", [
     (256, 128, 64, 0, 0, 1), (300, 70, 45, 0, 0, 1), (128, 256, 32, 0, 1, 1), (77, 130, 19, 0, 1, 1),
     (128, 128, 4096, 1, 0, 8), (480, 40, 1000, 1, 0, 4), (129, 129, 17, 1, 1, 1), (1024, 128, 1024, 0, 0, 1),
-    # full tiles in every layout (64-row and 128-row tiles of the kernel without bounds checks), with and without
-    # a split of the reduction, and a reduction too short for that kernel
+    # whole tiles in every layout: the short kernel (192 and 256 rows) and the split kernel (32 768 rows; with 32 parts
+    # of the reduction), and a reduction of two steps
     (192, 384, 208, 0, 0, 1), (192, 384, 208, 1, 0, 1), (192, 384, 208, 0, 1, 1), (192, 384, 208, 1, 1, 1),
     (32768, 256, 192, 0, 0, 1), (32768, 128, 192, 1, 0, 1), (32768, 256, 192, 0, 1, 1), (32768, 128, 192, 1, 1, 1),
     (256, 256, 16384, 1, 0, 8), (1024, 128, 8192, 1, 0, 32), (32768, 256, 64, 0, 1, 1),
-    # edge tiles read with whole 16-byte units (extents are multiples of the unit, not of the tile): the three
-    # products of a small hierarchy level, forward, weight gradient (with a cut last split) and projection gradient
+    # edge tiles, extents that are multiples of four and not of the tile: the three products of a small hierarchy
+    # level, forward, weight gradient (in the short kernel, and with a cut last split in the other) and projection
+    # gradient
     (346, 256, 1024, 0, 0, 1), (1024, 256, 346, 1, 0, 1), (346, 1024, 256, 0, 1, 1), (512, 128, 6844, 1, 0, 64),
     (200, 72, 104, 0, 0, 1), (200, 72, 104, 1, 1, 1), (36, 8, 12, 1, 0, 1)])
 def test_gemm_against_float64(rows, cols, inner, at, bt, split):
@@ -97,7 +98,8 @@ def test_gemm_at_even_edges_of_wide_tiles(rows, cols, inner, at, split):
     b = rng.normal(size=(inner, cols)).astype(np.float32)
     exp = (a.T if at else a).astype(np.float64) @ b.astype(np.float64)
     # the bound of the test above
-    assert np.linalg.norm(_gemm_f32(a, b, at, 0, split) - exp) / np.linalg.norm(exp) < np.sqrt(inner / 2 + 1) * 2.0 ** -24
+    error = np.linalg.norm(_gemm_f32(a, b, at, 0, split) - exp) / np.linalg.norm(exp)
+    assert error < np.sqrt(inner / 2 + 1) * 2.0 ** -24
 
 
 # reductions whose last step has eight, sixteen or twenty-four elements, alone and behind whole steps
@@ -185,8 +187,8 @@ def test_gemm_of_operands_with_long_rows(ld, at):
     wide = torch.empty(a.shape[0] * ld, dtype=torch.float32, device=DEV)
     wide.as_strided(a.shape, (ld, 1)).copy_(t(a))
     tb, tc = t(b), torch.full((rows, cols), float("nan"), device=DEV)
-    _lib.call("pccnn_gemm_f32", _lib.P(wide.data_ptr()), _lib.P(tb.data_ptr()), _lib.P(tc.data_ptr()), rows, cols, inner,
-              at, 0, ld, cols, cols, 1, 0, 0, 0, 1, None, 0, _lib.P(torch.cuda.current_stream().cuda_stream))
+    _lib.call("pccnn_gemm_f32", _lib.P(wide.data_ptr()), _lib.P(tb.data_ptr()), _lib.P(tc.data_ptr()), rows, cols,
+              inner, at, 0, ld, cols, cols, 1, 0, 0, 0, 1, None, 0, _lib.P(torch.cuda.current_stream().cuda_stream))
     assert relerr(tc.cpu().numpy(), (a.T if at else a).astype(np.float64) @ b.astype(np.float64)) < 1e-5
 
 
@@ -216,7 +218,7 @@ def test_gemm_of_non_finite_values_in_every_layout(rows, cols, inner, at, bt):
 
 @pytest.mark.parametrize("m,mlps,inner,co", [(200, 2, 48, 24), (256, 2, 208, 128), (32768, 3, 192, 128)])
 def test_gemm_batched_strided(m, mlps, inner, co):
-    # the second and third shapes have full tiles: the kernel without bounds checks, 64-row and 128-row tiles
+    # the first two shapes: the short kernel, at edges and with whole tiles; the third: the split kernel, whole tiles
     from pccnn_lib_amd import _lib
     rng = np.random.default_rng(0)
     a = rng.normal(size=(m, mlps * inner)).astype(np.float32)
@@ -370,7 +372,8 @@ def test_forward_projection_at_the_edges_of_its_tiles(ops, oracle, k, c_in):
 @pytest.mark.parametrize("n,m,per,c_in,k", [(5, 700, 3, 33, 15), (3, 400, 2, 64, 16), (7, 300, 1, 129, 8),
                                             (40, 900, 4, 70, 15), (2, 130, 1, 50, 33)])
 def test_feature_gradients_of_points_with_many_pairs(ops, oracle, n, m, per, c_in, k):
-    """Few points and many samples (a decoder's way up), on both sides of 64 pairs to a point; odd row widths."""
+    """Few points and few samples (a small decoder's way up), on both sides of 64 pairs to a point; odd row widths.  One
+    array of gradients: the copies per XCD begin at 2^23 pair features, see the next test."""
     rng = np.random.default_rng(n * m + c_in)
     pts = rng.uniform(0.0, 0.2, (n, 3)).astype(np.float32)
     smp = rng.uniform(0.0, 0.2, (m, 3)).astype(np.float32)
@@ -390,8 +393,10 @@ def test_feature_gradients_of_points_with_many_pairs(ops, oracle, n, m, per, c_i
             assert relerr(a.cpu().numpy(), e) < GRAD_TOL, name
 
 
-# on both sides of 2^23 pair features, odd row widths, with and without a gradient of the weights
-@pytest.mark.parametrize("n,m,c_in,k", [(333, 42366, 33, 5), (701, 42367, 33, 16), (90, 12000, 129, 9), (1000, 11000, 128, 8)])
+# one array of gradients and its copies per XCD, on both sides of 2^23 pair features; odd row widths, with and without a
+# gradient of the weights (which reads the projection that the copies then take the place of)
+@pytest.mark.parametrize("n,m,c_in,k", [(333, 42366, 33, 5), (701, 42367, 33, 16), (90, 12000, 129, 9),
+                                           (1000, 11000, 128, 8)])
 def test_feature_gradients_of_few_points_and_millions_of_pair_features(ops, oracle, n, m, c_in, k):
     rng = np.random.default_rng(n + m)
     per = 6
